@@ -9,13 +9,16 @@
 //   each 32-head warp adds its partials with an xor butterfly (16, 8, 4, 2, 1),
 //   warp 0 combines the warp sums with an xor butterfly over 8 lanes (4, 2, 1;
 //   lanes past the last warp hold 0.0f).
-// Here one thread scores one key (the key row in registers, the query in LDS)
-// and evaluates the same tree: a butterfly's lane-0 result is a balanced
-// binary tree whose leaves, left to right, are the heads in bit-reversed
-// order (h, h + 16, h + 8, h + 24, ...), so feeding the products in that
-// order to a five-level carry chain (HeadTree) adds exactly the reference's
-// pairs. Floating-point contraction is off in this file: every product and
-// sum rounds where the reference's does; the dot chains call fmaf.
+// The dot chains run on the matrix cores: v_mfma_f32_16x16x4_f32 adds its
+// four products to the accumulator one fma at a time, k ascending (checked bit
+// for bit against fmaf, denormals, infinities and cancellation included), so
+// 32 of them over d are the reference's chain. A butterfly's lane-0 result is
+// a balanced binary tree, which is added with the same pairs: heads h and
+// h + 16 are two accumulators of a lane, the rest are lane exchanges.
+// head_dim < 128 takes one thread per key, the tree fed in leaf order (heads
+// bit-reversed: h, h + 16, h + 8, h + 24, ...) to a carry chain (HeadTree).
+// Floating-point contraction is off in this file: every product and sum
+// rounds where the reference's does.
 //
 // Selection (cuda/indexer_allowed.cu:200-279): top_k rounds of argmax with
 // ties to the lowest index select exactly the top_k entries in
@@ -40,9 +43,7 @@ namespace {
 
 constexpr int kMaxHeads = 64;
 constexpr int kMaxDim = 128;
-constexpr int kQStride = kMaxDim + 4;   // query row stride in LDS for the four-thread form
 constexpr int kBins = 2048;
-constexpr int kBatchKeys = 128;   // keys per workgroup of the four-lane scorer
 constexpr int kSmallSelect = 16384;   // candidates one workgroup selects in LDS (the batched select's limit)
 
 __device__ inline unsigned ord_key(float s) {
@@ -56,40 +57,6 @@ __device__ inline float key_elem(const void *keys, size_t i) {
     if (kKind == 0) return static_cast<const float *>(keys)[i];
     if (kKind == 1) return f16_bits_to_f32(static_cast<const uint16_t *>(keys)[i]);
     return bf16_to_f32(static_cast<const uint16_t *>(keys)[i]);
-}
-
-// Copies the n_head x 128 fp32 query into LDS with all loads issued before
-// any store (a plain strided loop waits for each load in turn).
-template <int kStride = kMaxDim>
-__device__ inline void stage_query(float *qs, const float *q, int n_head) {
-    if (reinterpret_cast<uintptr_t>(q) & 15) {   // unaligned caller buffer: plain copy
-        for (int i = threadIdx.x; i < n_head * kMaxDim; i += 256)
-            qs[(i / kMaxDim) * kStride + i % kMaxDim] = q[i];
-        return;
-    }
-    const int n4 = n_head * kMaxDim / 4;
-    float4_t v[kMaxHeads * kMaxDim / 4 / 256];
-#pragma unroll
-    for (int i = 0; i < kMaxHeads * kMaxDim / 4 / 256; ++i) {
-        const int k = (int)threadIdx.x + 256 * i;
-        v[i] = reinterpret_cast<const float4_t *>(q)[min(k, n4 - 1)];   // clamped: no branch between the loads
-    }
-#pragma unroll
-    for (int i = 0; i < kMaxHeads * kMaxDim / 4 / 256; ++i) {
-        const int k = (int)threadIdx.x + 256 * i;
-        if (k < n4)
-            *reinterpret_cast<float4_t *>(qs + (k / (kMaxDim / 4)) * kStride + 4 * (k % (kMaxDim / 4))) = v[i];
-    }
-}
-
-// Zero query rows and weights for the heads past n_head up to the next
-// multiple of 32 (a whole warp of the reference's block). Their products are
-// replaced by 0.0f anyway, as the reference's idle threads contribute.
-__device__ inline void pad_heads(float *qs, float *ws, int n_head, int stride = kMaxDim) {
-    const int n32 = (n_head + 31) & ~31;
-    for (int i = threadIdx.x; i < (n32 - n_head) * kMaxDim; i += 256)
-        qs[(n_head + i / kMaxDim) * stride + i % kMaxDim] = 0.0f;
-    if ((int)threadIdx.x < n32 - n_head) ws[n_head + threadIdx.x] = 0.0f;
 }
 
 // The reference's head sum (see the top of the file), fed one leaf at a time
@@ -126,193 +93,177 @@ struct HeadTree {
 __device__ inline int head_of_leaf(int t) {
     return (t & ~31) | (int)(__builtin_bitreverse32((unsigned)(t & 31)) >> 27);
 }
-// First head of four-head group g: the 3 low bits of g reversed.
-__device__ inline int head_of_group(int g) {
-    return (g & ~7) * 4 + (int)(__builtin_bitreverse32((unsigned)(g & 7)) >> 29);
-}
-
 // relu and the rounded product of one head (cuda/indexer_allowed.cu:89-90)
 __device__ inline float head_partial(float dot, float w) {
     if (dot < 0.0f) dot = 0.0f;
     return dot * w;
 }
 
-// head_dim 128, one key per thread, the key row in registers as fp32 and the
-// query and the weights in LDS: every multiply-add takes its query value from
-// a broadcast 16-byte LDS read (in-order returns, so the reads run several
-// steps ahead of their use). Two heads at a time: their dot chains are
-// independent, and the chains and the head sum keep the canonical order.
+// ---- head_dim 128: scores on the fp32 matrix cores -----------------------------------------
+
+constexpr int kTileKeys = 16;             // keys per 16x16x4 tile
+constexpr int kRowStride = kMaxDim + 4;   // staged row in LDS: the 16 rows x 4 lane groups of a step on all banks
+
+// Rows [r0, r0 + 16) of 128 elements (rows past `last` repeat it), two
+// 16-byte loads (fp32) or one per thread of a 256-thread workgroup, widened
+// to fp32 in LDS rows by put. `wide`: the base is 16-byte aligned; else the
+// elements are read one by one.
 template <int kKind>
-__device__ __attribute__((always_inline)) inline float score_lds(const float *qs, const float *ws,
-                                                                 const void *__restrict__ keys,
-                                                                 int c, int n_head) {
-    float k[kMaxDim];
-    if (kKind == 0) {
-        const float4_t *src = reinterpret_cast<const float4_t *>(
-            static_cast<const float *>(keys) + (size_t)c * kMaxDim);
+struct TileLoad {
+    static constexpr int kPer = kKind == 0 ? 4 : 8;                       // elements per 16 bytes
+    static constexpr int kLoads = kTileKeys * kMaxDim / kPer / 256;       // 2 or 1
+    uint4_t raw[kLoads];
+    __device__ inline void load(const void *base, long long r0, long long last, bool wide) {
 #pragma unroll
-        for (int v = 0; v < kMaxDim / 4; ++v) {
-            const float4_t u = src[v];
+        for (int u = 0; u < kLoads; ++u) {
+            const int v = (int)threadIdx.x + 256 * u;
+            const long long r = r0 + v / (kMaxDim / kPer);
+            const size_t i = (size_t)(r < last ? r : last) * kMaxDim + (v % (kMaxDim / kPer)) * kPer;
+            if (kKind == 0) {
+                const uint32_t *p = static_cast<const uint32_t *>(base) + i;
+                raw[u] = wide ? *reinterpret_cast<const uint4_t *>(p) : uint4_t{p[0], p[1], p[2], p[3]};
+            } else {
+                const uint16_t *p = static_cast<const uint16_t *>(base) + i;
+                if (wide) raw[u] = *reinterpret_cast<const uint4_t *>(p);
+                else
 #pragma unroll
-            for (int e = 0; e < 4; ++e) k[4 * v + e] = u[e];
-        }
-    } else {
-        const uint4_t *src = reinterpret_cast<const uint4_t *>(
-            static_cast<const uint16_t *>(keys) + (size_t)c * kMaxDim);
-#pragma unroll
-        for (int v = 0; v < kMaxDim / 8; ++v) {
-            const uint4_t u = src[v];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const uint16_t h = (uint16_t)((u[e >> 1] >> (16 * (e & 1))) & 0xFFFF);
-                k[8 * v + e] = kKind == 1 ? f16_bits_to_f32(h) : bf16_to_f32(h);
+                    for (int k = 0; k < 4; ++k) raw[u][k] = (uint32_t)p[2 * k] | (uint32_t)p[2 * k + 1] << 16;
             }
         }
     }
-    // four heads at a time (four independent dot chains keep the VALU busy):
-    // group g = heads h, h + 16, h + 8, h + 24 of one warp, whose products
-    // the butterfly's first two levels add as ((p_h + p_h+16) + (p_h+8 + p_h+24))
-    HeadTree<3> tree;
-    const int n_groups = ((n_head + 31) & ~31) / 4;
-    for (int g = 0; g < n_groups; ++g) {
-        const int h = head_of_group(g);
-        float v = 0.0f;
-        if (h < n_head) {   // else all four heads are idle threads of the reference
-            const float4_t *q0 = reinterpret_cast<const float4_t *>(qs + h * kMaxDim);
-            constexpr int kOff[4] = {0, 16, 8, 24};
-            float d[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-            // the query reads run kAhead steps ahead of their use (LDS returns
-            // in order; with two waves per SIMD nothing else hides the latency)
-            constexpr int kAhead = 3;
-            float4_t a[kAhead][4];
+    __device__ inline void put(float *rows) const {
 #pragma unroll
-            for (int v4 = 0; v4 < kAhead; ++v4)
+        for (int u = 0; u < kLoads; ++u) {
+            const int v = (int)threadIdx.x + 256 * u;
+            float *d = rows + (v / (kMaxDim / kPer)) * kRowStride + (v % (kMaxDim / kPer)) * kPer;
+            float f[kPer];
 #pragma unroll
-                for (int z = 0; z < 4; ++z) a[v4][z] = q0[kOff[z] * (kMaxDim / 4) + v4];
-#pragma unroll
-            for (int v4 = 0; v4 < kMaxDim / 4; ++v4) {
-                float4_t cur[4];
-#pragma unroll
-                for (int z = 0; z < 4; ++z) cur[z] = a[v4 % kAhead][z];
-                if (v4 + kAhead < kMaxDim / 4) {
-#pragma unroll
-                    for (int z = 0; z < 4; ++z) a[v4 % kAhead][z] = q0[kOff[z] * (kMaxDim / 4) + v4 + kAhead];
-                }
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-#pragma unroll
-                    for (int z = 0; z < 4; ++z) d[z] = fmaf(cur[z][e], k[4 * v4 + e], d[z]);
+            for (int e = 0; e < kPer; ++e) {
+                const uint16_t h = (uint16_t)((raw[u][e * 4 / kPer] >> (16 * (e & 1))) & 0xFFFF);
+                f[e] = kKind == 0 ? __uint_as_float(raw[u][e & 3]) : (kKind == 1 ? f16_bits_to_f32(h) : bf16_to_f32(h));
             }
-            float p[4];
 #pragma unroll
-            for (int z = 0; z < 4; ++z) {
-                // heads past n_head give +0.0f (the reference's idle threads);
-                // their query rows and weights are zero-padded, so the loads
-                // stay in bounds, and a bit mask replaces the product
-                const float pz = head_partial(d[z], ws[h + kOff[z]]);
-                p[z] = __int_as_float(__float_as_int(pz) & (h + kOff[z] < n_head ? ~0 : 0));
-            }
-            v = (p[0] + p[1]) + (p[2] + p[3]);
+            for (int e = 0; e < kPer; e += 4)
+                *reinterpret_cast<float4_t *>(d + e) = float4_t{f[e], f[e + 1], f[e + 2], f[e + 3]};
         }
-        tree.push(g, v);
     }
-    return tree.result();
+};
+
+// Sum over the lanes l % 16 of a value per lane, with the butterfly's offsets
+// 8, 4, 2, 1 (row rotations: after the 8 step a lane's value repeats every 8
+// lanes, so a rotation by 4 pairs the lanes of an xor by 4; then quads).
+__device__ inline float lanes16_sum(float v) {
+    v = v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xF, 0xF, false));
+    v = v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xF, 0xF, false));
+    v = v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xF, 0xF, false));
+    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, false));
 }
 
-// head_dim 128 with four threads per key (adjacent lanes): thread `part`
-// holds dims [32 part, 32 part + 32) of the key and continues the dot chain of
-// part - 1 (handed over by a lane shift), so every head's dot is still one fma
-// chain over d ascending from +0, and part 3 runs the head sum in head order:
-// bit-identical to the one-thread form, with a quarter of the key registers
-// (several waves per SIMD hide the LDS latency of the query reads). In
-// iteration i, part p works on head i - p. The query rows sit kQStride floats
-// apart in LDS: with stride 128 the four parts' reads (offsets 32 p - 128 p)
-// would fall on the same banks; 132 spreads them over four bank groups.
-// load_key32 reads one part's dims.
-template <int kKind>
-__device__ inline void load_key32(const void *__restrict__ keys, int c, int part, float *k) {
-    if (kKind == 0) {
-        const float4_t *src = reinterpret_cast<const float4_t *>(
-            static_cast<const float *>(keys) + (size_t)c * kMaxDim + 32 * part);
+// One sequence's keys and where its scores go.
+struct ScoreSeq {
+    const float *q, *w;      // [n_head][128], [n_head]
+    const void *keys;
+    long long row0;          // first key row
+    float *scores;           // of key 0
+    int n;
+};
+
+// Scores keys [c0, end) of one sequence by a workgroup of four waves, 16 a
+// time: wave t takes heads 16 t .. 16 t + 15 (32 registers of query operands
+// and one accumulator), and the products meet in LDS for the tree. Heads past
+// n_head read head 0 and add +0.0f, as the reference's idle threads do.
+// store(key, score) is called by the lane that finished the key.
+//
+// What bounds it: the fp32 matrix rate, 15 ns per 16 keys x 16 heads x 4 dims
+// and SIMD, to which every vector instruction adds its own time (fp32 MFMAs
+// and VALU use the same units, measured). So the keys are widened once per
+// workgroup into LDS rows, from which LDS reads bring the step operands; the
+// next keys' loads and stores ride along, with one barrier per 16 keys. The
+// query goes through LDS too, as whole rows: operand-wise 4-byte loads of it
+// took 9 us of a 35k-key launch. Measured (64 heads, kernel alone): 131072
+// bf16 keys 46.0 -> 34.1 us against one fma chain per thread, 35k fp32 keys
+// of 16 sequences 22.4 -> 11.1 us against four chained lanes per key, and
+// against a lane per head 5.2 / 8.5 / 11.7 / 18.2 -> 4.5 / 4.6 / 5.8 / 6.8 us
+// at 1100 / 3000 / 6000 / 10000 keys, so one form serves every size.
+//
+// lds: kScoreLds floats, holding the query rows while they become operands,
+// then the key tiles, the products and (hist) the caller's level-1 histogram,
+// which is cleared here.
+constexpr int kTileLds = kTileKeys * kRowStride;
+constexpr int kScoreLds = 4 * kTileLds;                     // 33 KB: four workgroups per CU
+constexpr int kPartAt = 2 * kTileLds, kHistAt = kPartAt + 2 * 4 * 4 * 64;
+static_assert(kHistAt + kBins <= kScoreLds, "score LDS");
+template <int kKind, class F>
+__device__ inline void score_keys(const ScoreSeq &S, int n_head, int c0, int end, float *lds, bool hist, F store) {
+    const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4, t = threadIdx.x >> 6;
+    const bool wide = (reinterpret_cast<uintptr_t>(S.keys) & 15) == 0;
+    const long long last = S.row0 + S.n - 1;
+    TileLoad<kKind> next;
+    next.load(S.keys, S.row0 + c0, last, wide);
+    const int h = 16 * t + col;
+    const bool live = h < n_head;
+    const float w = live ? S.w[h] : 0.0f;
+    // this wave's 16 query rows through its quarter of lds (whole rows per
+    // load: strided 4-byte loads of the operands cost more than the scoring)
+    float q[kMaxDim / 4];
+    {
+        float *mine = lds + t * kTileLds;
+        const bool wq = (reinterpret_cast<uintptr_t>(S.q) & 15) == 0;
+        float4_t v[kTileKeys * kMaxDim / 4 / 64];
 #pragma unroll
-        for (int v = 0; v < 8; ++v) {
-            const float4_t u = src[v];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) k[4 * v + e] = u[e];
+        for (int u = 0; u < kTileKeys * kMaxDim / 4 / 64; ++u) {
+            const int i = lane + 64 * u, r = min(16 * t + i / (kMaxDim / 4), n_head - 1);
+            const float *p = S.q + (size_t)r * kMaxDim + 4 * (i % (kMaxDim / 4));
+            v[u] = wq ? *reinterpret_cast<const float4_t *>(p) : float4_t{p[0], p[1], p[2], p[3]};
         }
-    } else {
-        const uint4_t *src = reinterpret_cast<const uint4_t *>(
-            static_cast<const uint16_t *>(keys) + (size_t)c * kMaxDim + 32 * part);
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const uint4_t u = src[v];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const uint16_t h = (uint16_t)((u[e >> 1] >> (16 * (e & 1))) & 0xFFFF);
-                k[8 * v + e] = kKind == 1 ? f16_bits_to_f32(h) : bf16_to_f32(h);
-            }
+        for (int u = 0; u < kTileKeys * kMaxDim / 4 / 64; ++u) {
+            const int i = lane + 64 * u;
+            *reinterpret_cast<float4_t *>(mine + (i / (kMaxDim / 4)) * kRowStride + 4 * (i % (kMaxDim / 4))) = v[u];
         }
+#pragma unroll
+        for (int i = 0; i < kMaxDim / 4; ++i) q[i] = mine[col * kRowStride + 4 * i + g];
+    }
+    __syncthreads();   // lds changes its use
+    unsigned *lh = reinterpret_cast<unsigned *>(lds + kHistAt);
+    if (hist)
+        for (int i = threadIdx.x; i < kBins; i += 256) lh[i] = 0;
+    next.put(lds);
+    if (c0 + kTileKeys < end) next.load(S.keys, S.row0 + c0 + kTileKeys, last, wide);
+    __syncthreads();
+    for (int buf = 0; c0 < end; c0 += kTileKeys, buf ^= 1) {
+        const float *kr = lds + buf * kTileLds + col * kRowStride + g;
+        float *part = lds + kPartAt + buf * (4 * 4 * 64) + lane;   // [wave][i][lane]
+        float k[kMaxDim / 4];
+#pragma unroll
+        for (int i = 0; i < kMaxDim / 4; ++i) k[i] = kr[4 * i];
+        if (c0 + kTileKeys < end) {
+            next.put(lds + (buf ^ 1) * kTileLds);
+            if (c0 + 2 * kTileKeys < end) next.load(S.keys, S.row0 + c0 + 2 * kTileKeys, last, wide);
+        }
+        float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < kMaxDim / 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i], q[i], acc, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)   // key 4 g + i
+            part[(4 * t + i) * 64] = __int_as_float(__float_as_int(head_partial(acc[i], w)) & (live ? ~0 : 0));
+        // the only barrier: the other buffers are written again after the
+        // next one, by when their readers are past it
+        __syncthreads();
+        // wave t finishes key 4 g + t of each lane group
+        const float w0 = lanes16_sum(part[t * 64] + part[(4 + t) * 64]);
+        const float w1 = lanes16_sum(part[(8 + t) * 64] + part[(12 + t) * 64]);
+        const int c = c0 + 4 * g + t;
+        // warp 0's 8-lane butterfly over (w0, w1, 0, ..., 0)
+        if (col == 0 && c < S.n) store(c, (w0 + 0.0f) + (w1 + 0.0f));
     }
 }
 
-// Two keys (c0, c1) per group of four lanes: their chains are independent,
-// which gives the VALU two dependency chains to interleave. The group runs
-// kLeaves consecutive leaves (heads, in bit-reversed order within their
-// warp), from leaf0, of the reference's block (a whole warp: 32), and part 3
-// returns their subtree of the warp's butterfly for both keys.
-template <int kKind, int kLeaves>
-__device__ __attribute__((always_inline)) inline void score_chain4x2(const float *qs, const float *ws,
-                                                                     const void *__restrict__ keys,
-                                                                     int c0, int c1, int n_head, int part,
-                                                                     float *pbuf, int kl0, int kl1, int leaf0,
-                                                                     float &w0, float &w1) {
-    float k0[32], k1[32];
-    load_key32<kKind>(keys, c0, part, k0);
-    load_key32<kKind>(keys, c1, part, k1);
-    float carry0 = 0.0f, carry1 = 0.0f;
-    for (int i = 0; i < kLeaves + 3; ++i) {
-        const int leaf = leaf0 + i - part;
-        const bool in = i - part >= 0 && i - part < kLeaves;
-        const int h = in ? head_of_leaf(leaf) : 0;
-        const bool act = in && h < n_head;
-        const float4_t *qv = reinterpret_cast<const float4_t *>(qs + (act ? h : 0) * kQStride + 32 * part);
-        float d0 = part == 0 ? 0.0f : carry0;
-        float d1 = part == 0 ? 0.0f : carry1;
-#pragma unroll
-        for (int v = 0; v < 8; ++v) {
-            const float4_t a = qv[v];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                d0 = fmaf(a[e], k0[4 * v + e], d0);
-                d1 = fmaf(a[e], k1[4 * v + e], d1);
-            }
-        }
-        // lane l takes lane l-1's chains (row_shr:1; part 0 ignores them)
-        carry0 = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(d0), 0x111, 0xF, 0xF, false));
-        carry1 = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(d1), 0x111, 0xF, 0xF, false));
-        // the head's product, in leaf order, for the tree below
-        if (part == 3 && in) {
-            pbuf[leaf * kBatchKeys + kl0] = act ? head_partial(d0, ws[h]) : 0.0f;
-            pbuf[leaf * kBatchKeys + kl1] = act ? head_partial(d1, ws[h]) : 0.0f;
-        }
-    }
-    // In leaf order the butterfly of a warp of heads is a balanced tree of
-    // adjacent pairs.
-    if (part == 3) {
-#pragma unroll
-        for (int z = 0; z < 2; ++z) {
-            const int kl = z ? kl1 : kl0;
-            float v[kLeaves];
-#pragma unroll
-            for (int t = 0; t < kLeaves; ++t) v[t] = pbuf[(leaf0 + t) * kBatchKeys + kl];
-#pragma unroll
-            for (int n = kLeaves / 2; n >= 1; n >>= 1)
-#pragma unroll
-                for (int t = 0; t < n; ++t) v[t] = v[2 * t] + v[2 * t + 1];
-            (z ? w1 : w0) = v[0];
-        }
-    }
-}
+// Keys per workgroup (a multiple of 16) for n keys in all: one tile each up
+// to four workgroups per CU (what the LDS holds), beyond that more tiles
+// each, which spreads the query's staging over them.
+constexpr int kScoreBlocks = 1024;
+int score_keys_per_block(long long n) { return 16 * (int)((n + 16 * kScoreBlocks - 1) / (16 * kScoreBlocks)); }
 
 // Any head_dim <= 128: the key row is zero-padded to 128 in registers and
 // the query is read with the same padding from LDS.
@@ -341,55 +292,41 @@ __device__ inline float score_any(const float *qs, const float *ws, const void *
     return tree.result();
 }
 
-// kFull: head_dim == 128 (the scalar-load path); otherwise the LDS path. Two
-// instantiations so that neither path's registers limit the other's occupancy.
-// One key per thread: 131072 keys make two waves per SIMD, so the register
-// budget is that of two waves per SIMD, which holds the query reads several
-// steps ahead (measured 67 -> 61 us for the indexer over 131072 keys).
+// Scores of one sequence and, with hist, the level-1 histogram of the first
+// n_cand. kFull: head_dim == 128, keys_per_blk keys per workgroup; else one
+// thread per key with the query in LDS.
 template <int kKind, bool kFull>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void score_kernel(const float *__restrict__ q,
+__global__ __launch_bounds__(256) void score_kernel(const float *__restrict__ q,
                                                     const float *__restrict__ w,
                                                     const void *__restrict__ keys, int n_comp,
                                                     int n_head, int head_dim,
                                                     float *__restrict__ scores,
-                                                    unsigned *__restrict__ hist, int n_cand) {
-    __shared__ unsigned lh[kBins];
-    if (hist)
-        for (int i = threadIdx.x; i < kBins; i += 256) lh[i] = 0;
-    __shared__ __attribute__((aligned(16))) float qs[kMaxHeads * kQStride];
-    __shared__ float ws[kMaxHeads];
+                                                    unsigned *__restrict__ hist, int n_cand, int keys_per_blk) {
+    // kFull: lh is the histogram part of its LDS; else it follows the query
+    __shared__ __attribute__((aligned(16))) float lds[kFull ? kScoreLds : kMaxHeads * kMaxDim + kMaxHeads + kBins];
+    unsigned *lh = reinterpret_cast<unsigned *>(lds + (kFull ? kHistAt : kMaxHeads * kMaxDim + kMaxHeads));
     if (kFull) {
-        // one thread per key: the query staged once per 256 keys (the four-lane
-        // chained form measures slower here, where a launch has many keys)
-        const int c = blockIdx.x * 256 + threadIdx.x;
-        float s = 0.0f;
-        stage_query(qs, q, n_head);
-        for (int i = threadIdx.x; i < n_head; i += 256) ws[i] = w[i];
-        pad_heads(qs, ws, n_head);
-        __syncthreads();
-        if (c < n_comp) s = score_lds<kKind>(qs, ws, keys, c, n_head);
-        if (c < n_comp) scores[c] = s;
-        if (hist) {
-            __syncthreads();
-            if (c < n_cand) atomicAdd(&lh[ord_key(s) >> 21], 1u);
-            __syncthreads();
-            for (int i = threadIdx.x; i < kBins; i += 256)
-                if (lh[i]) atomicAdd(&hist[i], lh[i]);
-        }
-        return;
-    }
-    const int c = blockIdx.x * 256 + threadIdx.x;
-    float s = 0.0f;
-    {
+        const ScoreSeq S{q, w, keys, 0, scores, n_comp};
+        const int c0 = blockIdx.x * keys_per_blk;
+        score_keys<kKind>(S, n_head, c0, min(c0 + keys_per_blk, n_comp), lds, hist != nullptr, [&](int c, float s) {
+            scores[c] = s;
+            if (hist && c < n_cand) atomicAdd(&lh[ord_key(s) >> 21], 1u);
+        });
+    } else {
+        float *qs = lds, *ws = lds + kMaxHeads * kMaxDim;
+        if (hist)
+            for (int i = threadIdx.x; i < kBins; i += 256) lh[i] = 0;
         stage_to_lds(qs, q, n_head * head_dim);
         for (int i = threadIdx.x; i < n_head; i += 256) ws[i] = w[i];
         __syncthreads();
-        if (c < n_comp) s = score_any<kKind>(qs, ws, keys, c, n_head, head_dim);
+        const int c = blockIdx.x * 256 + threadIdx.x;
+        if (c < n_comp) {
+            const float s = score_any<kKind>(qs, ws, keys, c, n_head, head_dim);
+            scores[c] = s;
+            if (hist && c < n_cand) atomicAdd(&lh[ord_key(s) >> 21], 1u);
+        }
     }
-    if (c < n_comp) scores[c] = s;
     if (hist) {
-        __syncthreads();
-        if (c < n_cand) atomicAdd(&lh[ord_key(s) >> 21], 1u);
         __syncthreads();
         for (int i = threadIdx.x; i < kBins; i += 256)
             if (lh[i]) atomicAdd(&hist[i], lh[i]);
@@ -636,19 +573,20 @@ int launch_scores(const float *q, const float *w, const void *keys, int kind, in
                   int n_head, int head_dim, float *scores, unsigned *hist, int n_cand,
                   hipStream_t st) {
     const bool full = head_dim == kMaxDim;
-    const dim3 grid((n_comp + 255) / 256);
+    const int kpb = full ? score_keys_per_block(n_comp) : 256;
+    const dim3 grid((n_comp + kpb - 1) / kpb);
     switch (kind) {
     case 0:
-        if (full) hipLaunchKernelGGL((score_kernel<0, true>), grid, dim3(256), 0, st, q, w, keys, n_comp, n_head, head_dim, scores, hist, n_cand);
-        else hipLaunchKernelGGL((score_kernel<0, false>), grid, dim3(256), 0, st, q, w, keys, n_comp, n_head, head_dim, scores, hist, n_cand);
+        if (full) hipLaunchKernelGGL((score_kernel<0, true>), grid, dim3(256), 0, st, q, w, keys, n_comp, n_head, head_dim, scores, hist, n_cand, kpb);
+        else hipLaunchKernelGGL((score_kernel<0, false>), grid, dim3(256), 0, st, q, w, keys, n_comp, n_head, head_dim, scores, hist, n_cand, kpb);
         break;
     case 1:
-        if (full) hipLaunchKernelGGL((score_kernel<1, true>), grid, dim3(256), 0, st, q, w, keys, n_comp, n_head, head_dim, scores, hist, n_cand);
-        else hipLaunchKernelGGL((score_kernel<1, false>), grid, dim3(256), 0, st, q, w, keys, n_comp, n_head, head_dim, scores, hist, n_cand);
+        if (full) hipLaunchKernelGGL((score_kernel<1, true>), grid, dim3(256), 0, st, q, w, keys, n_comp, n_head, head_dim, scores, hist, n_cand, kpb);
+        else hipLaunchKernelGGL((score_kernel<1, false>), grid, dim3(256), 0, st, q, w, keys, n_comp, n_head, head_dim, scores, hist, n_cand, kpb);
         break;
     default:
-        if (full) hipLaunchKernelGGL((score_kernel<2, true>), grid, dim3(256), 0, st, q, w, keys, n_comp, n_head, head_dim, scores, hist, n_cand);
-        else hipLaunchKernelGGL((score_kernel<2, false>), grid, dim3(256), 0, st, q, w, keys, n_comp, n_head, head_dim, scores, hist, n_cand);
+        if (full) hipLaunchKernelGGL((score_kernel<2, true>), grid, dim3(256), 0, st, q, w, keys, n_comp, n_head, head_dim, scores, hist, n_cand, kpb);
+        else hipLaunchKernelGGL((score_kernel<2, false>), grid, dim3(256), 0, st, q, w, keys, n_comp, n_head, head_dim, scores, hist, n_cand, kpb);
         break;
     }
     return hip_status(hipGetLastError());
@@ -831,194 +769,42 @@ struct BatchArgs {
     const void *keys;          // key rows, sequence s at row key0[s]
     float *scores;             // same indexing as the key rows
     int32_t *pos_out;          // [n_seq][pos_stride]
-    int n_seq, n_head, top_k, n_recent, pos_stride;
+    int n_seq, n_head, top_k, n_recent, pos_stride, keys_per_blk;
     long long key0[kMaxSeq];
     int n_comp[kMaxSeq];
     int blk0[kMaxSeq + 1];     // first score block of each sequence
 };
 
-// kSplit threads per key (1 or 4); blocks of 256 threads cover 256 / kSplit keys.
-// Four chained lanes per key, two keys per lane group, 128 keys per
-// workgroup of 2 x 256 threads: thread group g runs the leaves of warp g of
-// the reference's block (heads 32 g .. 32 g + 31) for the same keys, so a
-// wave's chain is half as long and the launch has twice the waves (cfg-5
-// layer-step 195.5 -> 187.2 us; four groups of 16 leaves measured the same);
-// the two warp sums meet in LDS for warp 0's combine.
-constexpr int kGroups = 2;
-constexpr int kHalf = kBatchKeys / 2;            // a lane group's second key: kl + kHalf
-constexpr int kGroupThreads = 4 * kHalf;         // threads of one leaf group
-template <int kKind>
-__global__ __launch_bounds__(kGroupThreads * kGroups) void score_batch_kernel(const BatchArgs A) {
-    constexpr int kLeaves = kMaxHeads / kGroups;
+// The sequence of score workgroup blockIdx.x, and its first key there.
+__device__ inline ScoreSeq batch_seq(const BatchArgs &A, int keys_per_blk, int &c0) {
     int s = 0;
 #pragma unroll
     for (int i = 1; i < kMaxSeq; ++i)
         if (i < A.n_seq && (int)blockIdx.x >= A.blk0[i]) s = i;
-    int n = 0;
-    long long k0 = 0;
-#pragma unroll
-    for (int i = 0; i < kMaxSeq; ++i)
-        if (i == s) {
-            n = A.n_comp[i];
-            k0 = A.key0[i];
-        }
+    ScoreSeq S{};
     int first = 0;
 #pragma unroll
     for (int i = 0; i < kMaxSeq; ++i)
-        if (i == s) first = A.blk0[i];
-    const int grp = (int)threadIdx.x / kGroupThreads, tl = (int)threadIdx.x % kGroupThreads;
-    const int c = ((int)blockIdx.x - first) * kBatchKeys + tl / 4;
-    __shared__ __attribute__((aligned(16))) float qs[kMaxHeads * kQStride];
-    __shared__ float ws[kMaxHeads];
-    __shared__ float pbuf[kMaxHeads * kBatchKeys];   // [leaf][key of the block]
-    __shared__ float sub[kGroups][kBatchKeys];       // subtree sums per key of the block
-    const float *qg = A.q + (size_t)s * A.n_head * kMaxDim;
-    const float *wg = A.w + (size_t)s * A.n_head;
-    if (threadIdx.x < 256) stage_query<kQStride>(qs, qg, A.n_head);
-    for (int i = threadIdx.x; i < A.n_head; i += kGroupThreads * kGroups) ws[i] = wg[i];
-    __syncthreads();
-    const int part = tl % 4;
-    const int kl = tl / 4;   // the group's first key within the block; the second is kl + kHalf
-    const int c1 = c + kHalf;
-    const int n_leaves = (A.n_head + 31) & ~31;   // an absent warp 1 adds +0.0f
-    const int leaf0 = grp * kLeaves;
-    float s0 = 0.0f, s1 = 0.0f;
-    if (c < n && leaf0 < n_leaves)
-        score_chain4x2<kKind, kLeaves>(qs, ws, A.keys, (int)(k0 + c), (int)(k0 + (c1 < n ? c1 : c)), A.n_head,
-                                       part, pbuf, kl, kl + kHalf, leaf0, s0, s1);
-    if (part == 3) {
-        sub[grp][kl] = s0;
-        sub[grp][kl + kHalf] = s1;
-    }
-    __syncthreads();
-    if (grp == 0 && part == 3 && c < n) {
-#pragma unroll
-        for (int z = 0; z < 2; ++z) {
-            const int k = kl + kHalf * z;
-            const float w0 = sub[0][k], w1 = sub[1][k];
-            // warp 0's 8-lane butterfly over (w0, w1, 0, ..., 0)
-            if (z == 0 || c1 < n) A.scores[k0 + c + kHalf * z] = (w0 + 0.0f) + (w1 + 0.0f);
-        }
-    }
-}
-
-// Lane-per-head scorer (the reference's own layout, cuda/indexer_allowed.cu:
-// 68-171: one thread per head): lane h of a wave holds q_h in registers, the
-// block's keys sit in LDS as fp32 and are read by broadcast, and a wave scores
-// kHeadsKpw keys, two dot chains at a time. The head sum is the reference's
-// tree literally: an xor butterfly over each 32-lane half (offsets 16 .. 1),
-// then lane 0's and lane 32's warp sums combined as warp 0 combines them.
-// Many keys per launch need few registers per key; this form suits a few
-// thousand keys, where one thread per key would leave most CUs idle.
-// Two keys per wave (one pair of chains) gives the most workgroups; eight
-// measured 135 us slower per token over 43 layers at context 4096.
-constexpr int kHeadsKpw = 2;                    // keys per wave
-constexpr int kHeadsKpb = 4 * kHeadsKpw;        // keys per workgroup
-// Up to this many keys per launch. Measured (one sequence, 64 heads, fp32
-// keys): this form 5.2 / 8.6 / 12.4 / 22.0 us at 1500 / 3000 / 6000 / 12000
-// keys, the four-lane form 19.3 / 19.6 / 20.0 us at 3000 / 6000 / 12000.
-constexpr long long kHeadsMaxKeys = 10240;
-template <int kKind>
-__global__ __launch_bounds__(256) void score_heads_kernel(const BatchArgs A) {
-    int s = 0;
-#pragma unroll
-    for (int i = 1; i < kMaxSeq; ++i)
-        if (i < A.n_seq && (int)blockIdx.x >= A.blk0[i]) s = i;
-    int n = 0, first = 0;
-    long long k0 = 0;
-#pragma unroll
-    for (int i = 0; i < kMaxSeq; ++i)
         if (i == s) {
-            n = A.n_comp[i];
-            k0 = A.key0[i];
+            S.n = A.n_comp[i];
+            S.row0 = A.key0[i];
             first = A.blk0[i];
         }
-    const int c0 = ((int)blockIdx.x - first) * kHeadsKpb;
-    __shared__ __attribute__((aligned(16))) float qs[kMaxHeads * kQStride];
-    __shared__ __attribute__((aligned(16))) float ks[kHeadsKpb * kMaxDim];
-    const float *qg = A.q + (size_t)s * A.n_head * kMaxDim;
-    stage_query<kQStride>(qs, qg, A.n_head);
-    // the block's keys, widened to fp32 (rows past n are zeros, never stored):
-    // 16-byte loads, all issued before any is used (rows past n load row
-    // n - 1, so there is no branch between them)
-    constexpr int kEsz = kKind == 0 ? 4 : 2;
-    constexpr int kPer = 16 / kEsz;                    // elements per load
-    constexpr int kRowVecs = kMaxDim / kPer;
-    constexpr int kLoads = (kHeadsKpb * kRowVecs + 255) / 256;
-    const int rows_here = min(n - c0, kHeadsKpb);
-    const char *kbase = static_cast<const char *>(A.keys) + (size_t)(k0 + c0) * kMaxDim * kEsz;
-    if (rows_here > 0 && (reinterpret_cast<uintptr_t>(kbase) & 15) == 0) {
-        uint4_t kv[kLoads];
-#pragma unroll
-        for (int u = 0; u < kLoads; ++u) {
-            const int vi = (int)threadIdx.x + 256 * u;
-            const int kr = min(vi / kRowVecs, rows_here - 1);
-            kv[u] = reinterpret_cast<const uint4_t *>(kbase)[kr * kRowVecs + vi % kRowVecs];
-        }
-#pragma unroll
-        for (int u = 0; u < kLoads; ++u) {
-            const int vi = (int)threadIdx.x + 256 * u;
-            if (vi >= kHeadsKpb * kRowVecs) break;   // a block of few bf16 rows: fewer vectors than threads
-            const bool in = vi / kRowVecs < rows_here;
-            float f[kPer];
-#pragma unroll
-            for (int e = 0; e < kPer; ++e) {
-                const uint32_t w = kv[u][e * kEsz / 4];
-                const uint16_t h = (uint16_t)(e & 1 ? w >> 16 : w & 0xFFFF);
-                f[e] = kKind == 0 ? __uint_as_float(kv[u][e]) : (kKind == 1 ? f16_bits_to_f32(h) : bf16_to_f32(h));
-                f[e] = in ? f[e] : 0.0f;
-            }
-#pragma unroll
-            for (int e = 0; e < kPer; e += 4)
-                *reinterpret_cast<float4_t *>(ks + vi * kPer + e) = float4_t{f[e], f[e + 1], f[e + 2], f[e + 3]};
-        }
-    } else {
-        for (int i = threadIdx.x; i < kHeadsKpb * kMaxDim; i += 256) {
-            const int kr = i / kMaxDim, d = i % kMaxDim;
-            ks[i] = c0 + kr < n ? key_elem<kKind>(A.keys, (size_t)(k0 + c0 + kr) * kMaxDim + d) : 0.0f;
-        }
-    }
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int h = lane;
-    const bool live = h < A.n_head;
-    float q[kMaxDim];
-#pragma unroll
-    for (int v = 0; v < kMaxDim / 4; ++v) {
-        const float4_t t = *reinterpret_cast<const float4_t *>(qs + (live ? h : 0) * kQStride + 4 * v);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) q[4 * v + e] = t[e];
-    }
-    const float wh = live ? A.w[(size_t)s * A.n_head + h] : 0.0f;
-#pragma unroll 1
-    for (int kk = wave * kHeadsKpw; kk < (wave + 1) * kHeadsKpw; kk += 2) {
-        if (c0 + kk >= n) break;
-        float dot[2] = {0.0f, 0.0f};
-#pragma unroll
-        for (int v = 0; v < kMaxDim / 4; ++v) {
-            float4_t kv[2];
-#pragma unroll
-            for (int z = 0; z < 2; ++z) kv[z] = *reinterpret_cast<const float4_t *>(ks + (kk + z) * kMaxDim + 4 * v);
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int z = 0; z < 2; ++z) dot[z] = fmaf(q[4 * v + e], kv[z][e], dot[z]);
-        }
-#pragma unroll
-        for (int z = 0; z < 2; ++z) {
-            // idle heads (the reference's threads h >= n_head) add +0.0f
-            float v = __int_as_float(__float_as_int(head_partial(dot[z], wh)) & (live ? ~0 : 0));
-#pragma unroll
-            for (int off = 16; off > 0; off >>= 1) v = v + __shfl_xor(v, off);
-            const float w0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0));
-            const float w1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 32));
-            // warp 0's 8-lane butterfly over (w0, w1, 0, ...): lanes of an
-            // absent warp hold +0.0f, which (w1 + 0) reproduces
-            const float score = (w0 + 0.0f) + (w1 + 0.0f);
-            const int c = c0 + kk + z;
-            if (lane == 0 && c < n) A.scores[k0 + c] = score;
-        }
-    }
+    S.q = A.q + (size_t)s * A.n_head * kMaxDim;
+    S.w = A.w + (size_t)s * A.n_head;
+    S.keys = A.keys;
+    S.scores = A.scores + S.row0;
+    c0 = ((int)blockIdx.x - first) * keys_per_blk;
+    return S;
+}
+
+template <int kKind>
+__global__ __launch_bounds__(256) void score_batch_kernel(const BatchArgs A) {
+    __shared__ __attribute__((aligned(16))) float lds[kScoreLds];
+    int c0;
+    const ScoreSeq S = batch_seq(A, A.keys_per_blk, c0);
+    score_keys<kKind>(S, A.n_head, c0, min(c0 + A.keys_per_blk, S.n), lds, false,
+                      [&](int c, float s) { S.scores[c] = s; });
 }
 
 __device__ inline unsigned scan1024_excl(unsigned v, unsigned *wsum, unsigned *total) {
@@ -1425,14 +1211,10 @@ extern "C" int ds4hip_indexer_topk_positions_batch(
     A.top_k = top_k;
     A.n_recent = n_recent;
     A.pos_stride = pos_stride;
-    // Few keys in all: one wave per kHeadsKpw keys, lane = head
-    // (score_heads_kernel), which fills the chip where one group of lanes per
-    // key would not. Many keys: four chained lanes per key (score_batch_kernel).
     long long n_scored = 0;
     for (int s = 0; s < n_seq; ++s)
         if (n_comp_host[s] > top_k) n_scored += n_comp_host[s];
-    const bool heads = n_scored <= kHeadsMaxKeys;
-    const int keys_per_blk = heads ? kHeadsKpb : kBatchKeys;
+    const int keys_per_blk = A.keys_per_blk = score_keys_per_block(n_scored);
     int blk = 0;
     for (int s = 0; s < kMaxSeq; ++s) {
         const int n = s < n_seq ? n_comp_host[s] : 0;
@@ -1450,16 +1232,13 @@ extern "C" int ds4hip_indexer_topk_positions_batch(
         const dim3 g(blk), b(256);
         switch (key_kind) {
         case 0:
-            if (heads) hipLaunchKernelGGL(score_heads_kernel<0>, g, b, 0, st, A);
-            else hipLaunchKernelGGL(score_batch_kernel<0>, g, dim3(kGroupThreads * kGroups), 0, st, A);
+            hipLaunchKernelGGL(score_batch_kernel<0>, g, b, 0, st, A);
             break;
         case 1:
-            if (heads) hipLaunchKernelGGL(score_heads_kernel<1>, g, b, 0, st, A);
-            else hipLaunchKernelGGL(score_batch_kernel<1>, g, dim3(kGroupThreads * kGroups), 0, st, A);
+            hipLaunchKernelGGL(score_batch_kernel<1>, g, b, 0, st, A);
             break;
         default:
-            if (heads) hipLaunchKernelGGL(score_heads_kernel<2>, g, b, 0, st, A);
-            else hipLaunchKernelGGL(score_batch_kernel<2>, g, dim3(kGroupThreads * kGroups), 0, st, A);
+            hipLaunchKernelGGL(score_batch_kernel<2>, g, b, 0, st, A);
             break;
         }
     }
