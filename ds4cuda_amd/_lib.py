@@ -98,6 +98,9 @@ SIGNATURES: dict[str, list] = {
     "ds4hip_session_chunk_rows": [_vp, _i, _i, _i, _vp, _vp, _vp, _i, _vp, _i, _vp, _vp],
     "ds4hip_session_chunk_rows_host": [_vp, _i, _i, _i, _vp, _vp, _vp, _i, _vp, _i, _vp],
     "ds4hip_session_state_describe": [_vp, _i],
+    "ds4hip_session_chunk_step_workspace_bytes": [_vp, _i, _i],
+    "ds4hip_session_chunk_step": [_vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp],
+    "ds4hip_session_push_raw_rows": [_vp, _i, _vp, _i, _vp],
     "ds4hip_session_save_to_disk": [_vp, _vp, _i, C.c_char_p],
     "ds4hip_session_load_from_disk": [_vp, C.c_char_p, C.POINTER(_i), C.POINTER(_i)],
     "ds4hip_ds4cudak_probe": [C.c_char_p, _vp],
@@ -109,6 +112,7 @@ SIGNATURES: dict[str, list] = {
 RESTYPES = {"ds4hip_indexer_select_scratch_bytes": C.c_size_t,
             "ds4hip_flash_attn_prefill_fp8_workspace_size": C.c_size_t,
             "ds4hip_session_state_arena_bytes": C.c_size_t,
+            "ds4hip_session_chunk_step_workspace_bytes": C.c_size_t,
             "ds4hip_mul_mm_workspace_bytes": C.c_size_t,
             "ds4hip_compressor_batch_scratch_bytes": C.c_size_t,
             "ds4hip_attn_qkv_decode_workspace_bytes": C.c_size_t,

@@ -9,15 +9,15 @@ attention slice of one layer over the FP8 session (Session):
   1. the chunk's KV rows (Step 11) are quantized into the session's staging
      rows (one launch), so every token of the chunk can see the rows of the
      earlier chunk tokens while the ring still holds the window before p0;
-  2. per token, in position order, the steps whose state carries from one
-     token to the next: the attention compressor (and on ratio-4 layers the
-     indexer compressor) with their emitted rows appended to the session, and
-     on ratio-4 layers the indexer selection of the token's compressed rows
-     (Step 12, cuda/forward_layer.cu:997-1132);
+  2. the attention compressor (and on ratio-4 layers the indexer compressor)
+     of all tokens with their emitted rows appended to the session, and on
+     ratio-4 layers the indexer selection of each token's compressed rows
+     (Step 12, cuda/forward_layer.cu:997-1132), a few launches for the whole
+     chunk (ds4hip_session_chunk_step);
   3. one multi-problem FP8 decode launch computes all N tokens' attention
      (Step 13): token t attends the window rows still in the ring, staging
      rows 0..t and its compressed rows (ds4hip_session_chunk_rows);
-  4. the chunk's rows are pushed into the ring in order, which leaves the
+  4. the chunk's rows are pushed into the ring, which leaves the
      session exactly as N single-token steps would.
 
 Every kernel is a libds4hip.so entry point; torch provides device memory and
@@ -36,6 +36,12 @@ from .ops import _ptr, _stream
 N_HEAD, HEAD_DIM, N_ROT, IDX_DIM, N_EMBD = 64, 512, 64, 128, 4096
 CHUNK_MAX = 128
 INDEXER_TOP_K = 512
+
+
+class ChunkLayerArgs(C.Structure):
+    """ds4hip_chunk_layer (include/ds4hip_session.h)."""
+    _fields_ = [(k, C.c_void_p) for k in ("comp_kv", "comp_gate", "comp_ape", "comp_norm", "idx_kv", "idx_gate",
+                                          "idx_ape", "idx_norm", "idx_q_b", "idx_proj")] + [("top_k", C.c_int)]
 
 
 def _vp(x):
@@ -63,7 +69,7 @@ def forward_chunk_attn(session, il, p0, attn_norm, q_lora_norm, q_cur, kv_rope, 
     ops.attn_qkv_decode_f32 per token); sinks [64]; out [n, 64, 512] receives
     each token's attention output (Step 13's kqv). exact_p: the decode's P as
     f16 hi + lo (as Session.decode). Returns the workspace."""
-    from .ops import _check, decode_fp8_workspace_bytes, decode_opts
+    from .ops import _check, _dev, decode_fp8_workspace_bytes, decode_opts
     n = kv_rope.shape[0]
     if not 0 < n <= CHUNK_MAX:
         raise Ds4HipError("chunk of 1..128 tokens", -22)
@@ -83,59 +89,25 @@ def forward_chunk_attn(session, il, p0, attn_norm, q_lora_norm, q_cur, kv_rope, 
     # 1. the chunk's KV rows into the staging rows
     call("ds4hip_fp8_kv_quantize_append", _ptr(kv_rope), n, HEAD_DIM, N_ROT, _vp(s.codes), _vp(s.sexp),
          _vp(s.tail), C.c_longlong(s.n_cache_rows), None, st)
-    # 2. per token: compressors, emitted rows, indexer selection
+    # 2. compressors, emitted rows, indexer selection
     n_comp = np.zeros(n, np.int32)
     n_sel = np.zeros(n, np.int32)
     sel = None
     if ratio:
-        w = layer.w
-        coff = 2 if ratio == 4 else 1
-        emit = torch.empty(HEAD_DIM, device=dev)
-        kv_sc = torch.empty(2 * coff * HEAD_DIM, device=dev)
+        args = ChunkLayerArgs(top_k=layer.top_k)
+        names = ["comp_kv", "comp_gate", "comp_ape", "comp_norm"]
         if ratio == 4:
-            emit_i = torch.empty(IDX_DIM, device=dev)
-            kvi_sc = torch.empty(2 * coff * IDX_DIM, device=dev)
-            q_idx = torch.empty(N_HEAD * IDX_DIM, device=dev)
-            w_idx = torch.empty(N_HEAD, device=dev)
+            names += ["idx_kv", "idx_gate", "idx_ape", "idx_norm"]
+            if L.n_index_comp + (p0 + n) // ratio - p0 // ratio > layer.top_k:
+                names += ["idx_q_b", "idx_proj"]
             sel = torch.empty((n, layer.top_k), dtype=torch.int32, device=dev)
-            scores = torch.empty(max(L.cap_comp, 1), device=dev)
-            select = torch.empty(lib().ds4hip_indexer_select_scratch_bytes(max(L.cap_comp, 1)),
-                                 dtype=torch.uint8, device=dev)
-        for t in range(n):
-            pos = p0 + t
-            x = attn_norm[t]
-            e = C.c_int(0)
-            call("ds4hip_compressor_decode_step_f32_prealloc", 1, _ptr(x), _ptr(w["comp_kv"]),
-                 _ptr(w["comp_gate"]), _ptr(w["comp_ape"]), _ptr(w["comp_norm"]), N_EMBD, HEAD_DIM,
-                 ratio, pos, il, _vp(L.attn_state_kv), _vp(L.attn_state_score), _ptr(emit),
-                 C.byref(e), _ptr(kv_sc), _ptr(kv_sc[coff * HEAD_DIM:]), st)
-            if e.value:
-                session.push_comp(il, emit, stream=stream)
-            if ratio == 4:
-                ei = C.c_int(0)
-                call("ds4hip_compressor_decode_step_f32_prealloc", 0, _ptr(x), _ptr(w["idx_kv"]),
-                     _ptr(w["idx_gate"]), _ptr(w["idx_ape"]), _ptr(w["idx_norm"]), N_EMBD, IDX_DIM,
-                     ratio, pos, il, _vp(L.index_state_kv), _vp(L.index_state_score), _ptr(emit_i),
-                     C.byref(ei), _ptr(kvi_sc), _ptr(kvi_sc[coff * IDX_DIM:]), st)
-                if ei.value:
-                    session.push_index_comp(il, emit_i, stream=stream)
-            L = s.layers[il]
-            n_comp[t] = L.n_comp
-            n_sel[t] = L.n_comp
-            if ratio == 4 and L.n_index_comp > layer.top_k:
-                # indexer query and head weights of the token (Step 12b)
-                call("ds4hip_mul_mv_f16_f32", _ptr(w["idx_q_b"]), _ptr(q_lora_norm[t]), _ptr(q_idx),
-                     N_HEAD * IDX_DIM, 1024, st)
-                call("ds4hip_tail_rope_yarn_f32", _ptr(q_idx), _ptr(q_idx), N_HEAD, IDX_DIM, N_ROT, pos,
-                     il, st)
-                call("ds4hip_mul_mv_f16_f32", _ptr(w["idx_proj"]), _ptr(x), _ptr(w_idx), N_HEAD, N_EMBD,
-                     st)
-                call("ds4hip_scale_inplace_f32", _ptr(w_idx), N_HEAD,
-                     C.c_float(1.0 / np.sqrt(IDX_DIM * N_HEAD)), st)
-                call("ds4hip_indexer_topk_positions", _ptr(q_idx), _ptr(w_idx), _vp(L.index_comp_kv), 0,
-                     L.n_index_comp, N_HEAD, IDX_DIM, layer.top_k, 0, _ptr(scores), _ptr(select), None,
-                     _ptr(sel[t]), st)
-                n_sel[t] = layer.top_k
+        for k in names:
+            _dev(layer.w[k], k)
+            setattr(args, k, layer.w[k].data_ptr())
+        nb = lib().ds4hip_session_chunk_step_workspace_bytes(C.byref(s), il, n)
+        step_ws = torch.empty(max(nb, 1), dtype=torch.uint8, device=dev)
+        call("ds4hip_session_chunk_step", C.byref(s), il, p0, n, _ptr(attn_norm), _ptr(q_lora_norm), C.byref(args),
+             _ptr(sel), n_comp.ctypes.data_as(C.c_void_p), n_sel.ctypes.data_as(C.c_void_p), _ptr(step_ws), nb, st)
     # 3. all tokens' attention in one decode launch
     # list stride: the longest token list (window rows still in the ring, the
     # chunk's own rows up to the token, its compressed rows), from the layer's
@@ -168,7 +140,6 @@ def forward_chunk_attn(session, il, p0, attn_norm, q_lora_norm, q_cur, kv_rope, 
     # token-by-token loop leaves it
     if sel is not None and n_sel[-1] < n_comp[-1]:
         call("ds4hip_session_set_selection", C.byref(s), il, _ptr(sel[n - 1]), int(n_sel[-1]), st)
-    # 4. the chunk's rows into the ring, in position order
-    for t in range(n):
-        session.push_raw(il, kv_rope[t], stream=stream)
+    # 4. the chunk's rows into the ring
+    call("ds4hip_session_push_raw_rows", C.byref(s), il, _ptr(kv_rope), n, st)
     return workspace

@@ -224,5 +224,15 @@ int ds4hip_mm_kslice(int n_rows, int n_cols, int n_mats);
 int ds4hip_mm_f32_parts_mats(const float *const *W, float *const *part, const int *n_rows, const int *ks,
                              int n_mats, const float *X, int n_cols, int n_batch, hipStream_t st);
 
+// Top-k selections of a prompt chunk's tokens over one layer's indexer keys
+// (indexer.hip): token t sees the n_keys0 keys before the chunk and those its
+// tokens 0 .. t emit (one per `ratio` positions); a token with more than top_k
+// writes its selection to positions + t * top_k, the others nothing. scores:
+// scratch [n_tok][score_stride]. At most ds4hip_indexer_chunk_max_keys() keys.
+int ds4hip_indexer_chunk_max_keys();
+int ds4hip_indexer_chunk_topk(const float *q, const float *weights, const float *keys, int n_tok, int p0, int ratio,
+                              int n_keys0, int n_head, int top_k, float *scores, int score_stride,
+                              int32_t *positions, hipStream_t st);
+
 // Records the last failing status for the void-returning C++ shims.
 extern "C" int ds4hip_set_last_error(int code);

@@ -865,34 +865,23 @@ __device__ inline unsigned scan1024_small(unsigned v, unsigned *ws, unsigned *to
     return before + below;
 }
 
-__global__ __launch_bounds__(1024) void select_batch_kernel(const BatchArgs A) {
+// One 1024-thread workgroup selects of scores[0, n), n > top_k (see the top of
+// this section), and writes the positions to out.
+__device__ inline void select_body(const float *__restrict__ scores, int n, int top_k, int n_recent,
+                                   int32_t *__restrict__ out) {
     __shared__ unsigned keys[kSelMax];
     __shared__ __attribute__((aligned(16))) unsigned hist[2][256];
     __shared__ unsigned wemit[2][16];
-    const int s = blockIdx.x;
-    int n = 0;
-    long long k0 = 0;
-#pragma unroll
-    for (int i = 0; i < kMaxSeq; ++i)
-        if (i == s) {
-            n = A.n_comp[i];
-            k0 = A.key0[i];
-        }
-    int32_t *out = A.pos_out + (size_t)s * A.pos_stride;
     const int t = threadIdx.x;
-    if (n <= A.top_k) {
-        for (int i = t; i < n; i += 1024) out[i] = i;
-        return;
-    }
-    const int recent = A.n_recent < A.top_k ? A.n_recent : A.top_k;
+    const int recent = n_recent < top_k ? n_recent : top_k;
     const int n_cand = n - recent;
-    const unsigned need0 = (unsigned)(A.top_k - recent);
+    const unsigned need0 = (unsigned)(top_k - recent);
     // four loads in flight per thread (clamped, not branched): a strided copy
     // loop would wait for each load in turn
     for (int b = 0; b < n_cand; b += 4096) {
         unsigned v[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] = ord_key(A.scores[k0 + min(b + 1024 * u + t, n_cand - 1)]);
+        for (int u = 0; u < 4; ++u) v[u] = ord_key(scores[min(b + 1024 * u + t, n_cand - 1)]);
 #pragma unroll
         for (int u = 0; u < 4; ++u)
             if (b + 1024 * u + t < n_cand) keys[b + 1024 * u + t] = v[u];
@@ -968,6 +957,51 @@ __global__ __launch_bounds__(1024) void select_batch_kernel(const BatchArgs A) {
         }
     }
     for (int i = t; i < recent; i += 1024) out[tot_sel + i] = n_cand + i;
+}
+
+__global__ __launch_bounds__(1024) void select_batch_kernel(const BatchArgs A) {
+    const int s = blockIdx.x;
+    int n = 0;
+    long long k0 = 0;
+#pragma unroll
+    for (int i = 0; i < kMaxSeq; ++i)
+        if (i == s) {
+            n = A.n_comp[i];
+            k0 = A.key0[i];
+        }
+    int32_t *out = A.pos_out + (size_t)s * A.pos_stride;
+    if (n <= A.top_k) {
+        for (int i = threadIdx.x; i < n; i += 1024) out[i] = i;
+        return;
+    }
+    select_body(A.scores + k0, n, A.top_k, A.n_recent, out);
+}
+
+// ---- the tokens of a prompt chunk: one key list that grows along the chunk -----------------
+
+struct ChunkSelArgs {
+    const float *q, *w;        // [n][n_head][128], [n][n_head]
+    const float *keys;         // fp32 rows
+    float *scores;             // [n][stride]
+    int32_t *pos_out;          // [n][top_k]
+    int n_head, top_k, stride, keys_per_blk;
+    int n0, p0, ratio;         // keys before the chunk, its first position, tokens per key
+    __device__ inline int keys_of(int t) const { return n0 + (p0 + t + 1) / ratio - p0 / ratio; }
+};
+
+__global__ __launch_bounds__(256) void score_chunk_kernel(const ChunkSelArgs A) {
+    __shared__ __attribute__((aligned(16))) float lds[kScoreLds];
+    const int t = blockIdx.y, n = A.keys_of(t), c0 = (int)blockIdx.x * A.keys_per_blk;
+    if (n <= A.top_k || c0 >= n) return;
+    const ScoreSeq S{A.q + (size_t)t * A.n_head * kMaxDim, A.w + (size_t)t * A.n_head, A.keys, 0,
+                     A.scores + (size_t)t * A.stride, n};
+    score_keys<0>(S, A.n_head, c0, min(c0 + A.keys_per_blk, n), lds, false, [&](int c, float s) { S.scores[c] = s; });
+}
+
+__global__ __launch_bounds__(1024) void select_chunk_kernel(const ChunkSelArgs A) {
+    const int t = blockIdx.x, n = A.keys_of(t);
+    if (n <= A.top_k) return;
+    select_body(A.scores + (size_t)t * A.stride, n, A.top_k, 0, A.pos_out + (size_t)t * A.top_k);
 }
 
 // ---- two-launch selection of a long candidate list ----------------------------------------
@@ -1244,4 +1278,20 @@ extern "C" int ds4hip_indexer_topk_positions_batch(
     }
     hipLaunchKernelGGL(select_batch_kernel, dim3(n_seq), dim3(1024), 0, st, A);
     return ds4hip_set_last_error(hip_status(hipGetLastError()));
+}
+
+int ds4hip_indexer_chunk_max_keys() { return kSelMax; }
+
+int ds4hip_indexer_chunk_topk(const float *q, const float *weights, const float *keys, int n_tok, int p0, int ratio,
+                              int n_keys0, int n_head, int top_k, float *scores, int score_stride,
+                              int32_t *positions, hipStream_t st) {
+    ChunkSelArgs A{q, weights, keys, scores, positions, n_head, top_k, score_stride, 0, n_keys0, p0, ratio};
+    const int n_last = n_keys0 + (p0 + n_tok) / ratio - p0 / ratio;
+    if (n_last <= top_k) return 0;
+    if (n_last > kSelMax || n_last > score_stride) return kEINVAL;
+    A.keys_per_blk = score_keys_per_block((long long)n_last * n_tok);
+    hipLaunchKernelGGL(score_chunk_kernel, dim3((n_last + A.keys_per_blk - 1) / A.keys_per_blk, n_tok), dim3(256), 0,
+                       st, A);
+    hipLaunchKernelGGL(select_chunk_kernel, dim3(n_tok), dim3(1024), 0, st, A);
+    return hip_status(hipGetLastError());
 }

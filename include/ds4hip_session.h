@@ -179,6 +179,38 @@ int ds4hip_session_chunk_rows_host(const ds4hip_session_state *s, int il, int p0
                                    int sel_stride, int32_t *lists, int list_stride,
                                    long long *counts_out);
 
+/* Step 12 of a prompt chunk of a compressed layer (no counterpart in the
+ * reference, which runs it token by token, cuda/forward_batch.cu:264-284): the
+ * compressor steps of tokens p0 .. p0 + n_tok - 1 with their emitted rows and
+ * indexer keys appended to the session, and on indexer layers the selection of
+ * every token that sees more than top_k keys, at sel + t * top_k (device
+ * int32). Rows, keys, states and selections equal those of
+ * ds4hip_compressor_decode_step_f32, the pushes, ds4hip_mul_mv_f16_f32, the tail
+ * RoPE and ds4hip_indexer_topk_positions per token, bit for bit.
+ * n_comp_tok / n_sel_tok (host, n_tok each) receive the counts
+ * ds4hip_session_chunk_rows takes. attn_norm [n_tok][4096], q_lora_norm
+ * [n_tok][1024] (read only where a token selects, as idx_q_b, idx_proj and sel
+ * are). -28 when the emitted rows do not fit; a refused call changes nothing. */
+typedef struct ds4hip_chunk_layer {
+    const uint16_t *comp_kv, *comp_gate; /* [coff*512][4096] f16 (coff 2 at ratio 4, else 1) */
+    const uint16_t *comp_ape;            /* [ratio][coff*512] f16 */
+    const float *comp_norm;              /* [512] */
+    const uint16_t *idx_kv, *idx_gate;   /* [256][4096] f16, indexer layers */
+    const uint16_t *idx_ape;             /* [4][256] f16 */
+    const float *idx_norm;               /* [128] */
+    const uint16_t *idx_q_b;             /* [64*128][1024] f16 */
+    const uint16_t *idx_proj;            /* [64][4096] f16 */
+    int top_k;
+} ds4hip_chunk_layer;
+size_t ds4hip_session_chunk_step_workspace_bytes(const ds4hip_session_state *s, int il, int n_tok);
+int ds4hip_session_chunk_step(ds4hip_session_state *s, int il, int p0, int n_tok, const float *attn_norm,
+                              const float *q_lora_norm, const ds4hip_chunk_layer *w, int32_t *sel,
+                              int *n_comp_tok, int *n_sel_tok, void *workspace, size_t workspace_bytes,
+                              void *stream);
+
+/* ds4hip_session_push_raw for n_rows <= cap_raw rows [n_rows][512], in order. */
+int ds4hip_session_push_raw_rows(ds4hip_session_state *s, int il, const float *kv, int n_rows, void *stream);
+
 /* ---- disk format of the FP8 session (cuda/kv_persist.cuh:6-37, adapted) ---------- */
 
 /* One file holds the whole session: the header, then per layer its meta and
