@@ -13,22 +13,32 @@
 //   * QK^T: wave w owns rows [32w, 32w+32) (query w/2, heads 32(w&1)..) and
 //     computes S^T[32 keys x 32 rows] over all 512 dims with
 //     v_mfma_f32_16x16x32_f16 (A = K from LDS, B = Q^T held in registers);
-//   * softmax on its own rows (exp2 domain, lazy rescale: the reference
-//     max moves only when a row max exceeds it by 2^8);
+//   * softmax on its own rows (exp2 domain, relative to a reference fixed
+//     for the whole pass: the first tile's row max; a row that outgrows it
+//     sends its two queries to a second pass that starts from the row max);
 //   * P.V: wave w owns dims [128w, 128w+128) of all 128 rows (O: 256 fp32
 //     accumulators per lane), A = P from LDS (every wave's P tile is
 //     published there), B = V^T read from the same f16 tile with
 //     ds_read_b64_tr_b16.
 // The FP8 tile (32 rows x 584 B) is loaded into registers one tile ahead,
 // dequantized once per workgroup (v_cvt_scalef32_pk_f16_fp8) and written to a
-// double-buffered f16 LDS tile of 1056-byte rows whose 16-byte halves of each
+// triple-buffered f16 LDS tile of 1056-byte rows whose 16-byte halves of each
 // 32-byte column group swap on rows 8..15 of every 16 (row_swz). Inside a tile the keys are taken in the order pi (below):
 // the S^T rows of an MFMA, the P fragment and the V^T fragment then agree
 // without any register shuffling.
+//
+// A chunk of few queries would leave most CUs idle (one workgroup per two
+// queries), so its keys are split: `parts` workgroups per pair, each over its
+// own tiles with its own reference, and a merge of their (O, m, l). Parts are
+// chosen so that pairs x parts is at most one workgroup per CU, which bounds
+// the partials' workspace. Measured (one f16 P): 2 queries over
+// 8192 rows 495 -> 48 us, 20 over 4000 253 -> 44 us, 64 over 8000 494 -> 102
+// us, 255 over 2000 162 -> 107 us.
 
 #include "ds4hip_common.h"
 #include "../../include/ds4hip.h"
 
+#include <algorithm>
 
 using namespace ds4hip;
 
@@ -52,8 +62,11 @@ __device__ inline uint32_t row_swz(int r) {
 constexpr int kStageB = kTile * kRowB;
 constexpr int kRows = 128;           // query rows (2 queries x 64 heads) per workgroup
 constexpr float kLog2e = 1.4426950408889634f;
-constexpr float kRescale = 8.0f;     // fixup kernel: log2 slack before O is rescaled
-constexpr float kLazy = 15.0f;       // fast kernel: largest log2 growth of a row max (P <= 2^15)
+constexpr float kLazy = 15.0f;       // largest log2 growth of a row max in one pass (P <= 2^15)
+constexpr int kSplitWgs = 256;       // workgroups the split of a small chunk aims for
+constexpr int kMaxParts = 64;        // parts of a pair's keys
+constexpr int kCheckTiles = 6;       // tiles between looks at the reference
+constexpr int kMinPartTiles = 4;     // tiles of a part (a shorter one is mostly its prologue and its partial)
 
 struct PrefillArgs {
     const uint16_t *q;   // [n_q][64][512] bf16
@@ -62,7 +75,11 @@ struct PrefillArgs {
     const uint8_t *codes;
     const int8_t *sexp;
     const uint16_t *tail;
-    int *fail;           // [n_pairs] query pairs the fast kernel could not finish
+    int *fail;           // [pairs x parts] slots the first pass could not finish
+    float *row_max;      // [pairs x parts][128] their rows' maxima
+    float *part_o;       // [pairs x parts][128][512] unnormalized partials (parts > 1)
+    float *part_ml;      // [pairs x parts][2][128] their references and sums
+    int parts;
     int n_q;
     int n_cached;
     float kq_log2;
@@ -191,8 +208,7 @@ __device__ inline void load_q(const PrefillArgs &A, int qi, int w, int n16, int 
 // kPLo: P passed as f16 hi + lo halves (~22 bits, twice the P . V MFMAs);
 // otherwise one f16 with l summing the rounded P, so O stays an exactly
 // normalized average whose weights are off by at most 2^-11 relative.
-// The fixup kernel (prefill_fp8_kernel) always carries hi + lo.
-constexpr bool kPrefillPLo = true;
+// The second pass always carries hi + lo.
 
 template <bool kPLo>
 __device__ inline void pv_step(const half8_t (*phi)[64], const half8_t (*plo)[64], int lane,
@@ -226,211 +242,6 @@ __device__ inline void pv_step(const half8_t (*phi)[64], const half8_t (*plo)[64
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-    }
-}
-
-// Two-barrier form of the prefill. The launcher runs it as kFix = true, the
-// fixup kernel: only query pairs flagged by prefill_fast_kernel (a row max that
-// outgrew the fixed reference by more than 2^kLazy) run, and the reference max
-// moves whenever a row max exceeds it by 2^8, with O rescaled. kFix = false
-// (not launched) is the same pass with the fast kernel's fixed reference.
-// P is carried as f16 hi + lo (p - hi), so P . V keeps ~22 bits of P.
-template <bool kFix>
-__global__ __launch_bounds__(256) void prefill_fp8_kernel(const PrefillArgs A) {
-    __shared__ __attribute__((aligned(16))) uint8_t stages[2][kStageB];
-    __shared__ __attribute__((aligned(16))) half8_t phi[8][64];      // [row tile][lane]
-    __shared__ __attribute__((aligned(16))) half8_t plo[8][64];
-    __shared__ __attribute__((aligned(16))) float alpha_s[kRows];
-    __shared__ __attribute__((aligned(16))) int flag_s[4];
-    __shared__ __attribute__((aligned(16))) float fin_s[2][kRows];    // m, l per row
-
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int n16 = lane & 15, g = lane >> 4;
-    // heaviest query pairs first
-    const int pair = (int)gridDim.x - 1 - (int)blockIdx.x;
-    if (kFix && A.fail[pair] == 0) return;
-    const int q0 = 2 * pair;
-    const int qi = q0 + (w >> 1);                   // this wave's query
-    const bool q_ok = qi < A.n_q;
-    const int qpos = q_ok ? A.n_cached + qi : -1;   // last key this wave's rows see
-    const int n_all = A.n_cached + (q0 + 2 < A.n_q ? q0 + 2 : A.n_q);
-    const int n_tiles = (n_all + kTile - 1) / kTile;
-
-    // Q^T fragments: qf[rt][s] = Q[row 16rt+n16][dims 32s+8g .. +8]
-    half8_t qf[2][16];
-    load_q(A, q_ok ? qi : 0, w, n16, g, qf);
-
-    float4_t o[8][8];
-#pragma unroll
-    for (int a = 0; a < 8; ++a)
-#pragma unroll
-        for (int b = 0; b < 8; ++b) o[a][b] = float4_t{0, 0, 0, 0};
-    float m_use[2] = {-INFINITY, -INFINITY}, l_part[2] = {0.f, 0.f};
-    bool failed = false;
-
-    // lane-constant LDS offsets
-    uint32_t ka[2];           // QK A rows (key tile kt), dims 8g
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
-        const int r = pi_key(16 * kt + n16);
-        ka[kt] = r * kRowB + ((16 * g) ^ row_swz(r));
-    }
-    uint32_t va[2];           // V^T supplier rows (half h), dims 128w + 4(n16&3)
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int r = pi_key(16 * h + 4 * g + (n16 >> 2));
-        va[h] = r * kRowB + 256 * w + ((8 * (n16 & 3)) ^ row_swz(r));
-    }
-
-    Raw R;
-    load_raw(A, 0, n_all, tid, R);
-    store_tile(stages[0], tid, R);
-    load_raw(A, 1, n_all, tid, R);
-
-    int t = 0;
-    while (t < n_tiles) {
-        bool slow = false;
-        for (; t < n_tiles; ++t) {
-            lds_barrier();                                   // X: tile t is in stages[t&1]
-            // dequantize tile t+1 (past the end: zero rows, never read) and
-            // fetch tile t+2
-            store_tile(stages[(t + 1) & 1], tid, R);
-            load_raw(A, t + 2, n_all, tid, R);
-            const uint8_t *st = stages[t & 1];
-            // ---- S^T = K . Q^T ----
-            float4_t acc[2][2];
-#pragma unroll
-            for (int a = 0; a < 2; ++a)
-#pragma unroll
-                for (int b = 0; b < 2; ++b) acc[a][b] = float4_t{0, 0, 0, 0};
-#pragma unroll
-            for (int s = 0; s < 16; ++s) {
-                const int off = 64 * s;
-                const half8_t k0 = *reinterpret_cast<const half8_t *>(st + ka[0] + off);
-                const half8_t k1 = *reinterpret_cast<const half8_t *>(st + ka[1] + off);
-#pragma unroll
-                for (int rt = 0; rt < 2; ++rt) {
-                    acc[0][rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k0, qf[rt][s], acc[0][rt], 0, 0, 0);
-                    acc[1][rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k1, qf[rt][s], acc[1][rt], 0, 0, 0);
-                }
-            }
-            // ---- softmax on rows (rt, n16); lane holds keys pi(16kt+4g+r) ----
-            const bool edge = t * kTile + kTile - 1 > qpos;
-            bool need = false;
-#pragma unroll
-            for (int rt = 0; rt < 2; ++rt) {
-                float s2[2][4];
-                float mx = -INFINITY;
-#pragma unroll
-                for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        float v = acc[kt][rt][r] * A.kq_log2;
-                        if (edge && t * kTile + pi_key(16 * kt + 4 * g + r) > qpos) v = -INFINITY;
-                        s2[kt][r] = v;
-                        mx = fmaxf(mx, v);
-                    }
-                mx = xmax_16_32(mx);
-                float alpha = 1.0f;
-                if (m_use[rt] == -INFINITY) {
-                    m_use[rt] = mx;              // first tile: O and l are still zero
-                } else if (kFix) {
-                    if (mx > m_use[rt] + kRescale) {
-                        alpha = __builtin_amdgcn_exp2f(m_use[rt] - mx);
-                        m_use[rt] = mx;
-                        need = true;
-                    }
-                } else if (mx > m_use[rt] + kLazy) {
-                    failed = true;
-                }
-                l_part[rt] *= alpha;
-                const float m = m_use[rt];
-                half8_t hi, lo;
-#pragma unroll
-                for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const float p = s2[kt][r] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(s2[kt][r] - m);
-                        const half_t h = (half_t)p;
-                        l_part[rt] += kPrefillPLo ? p : (float)h;
-                        hi[4 * kt + r] = h;
-                        lo[4 * kt + r] = (half_t)(p - (float)h);
-                    }
-                phi[2 * w + rt][lane] = hi;
-                if (kPrefillPLo) plo[2 * w + rt][lane] = lo;
-                if (kFix && g == 0) alpha_s[32 * w + 16 * rt + n16] = alpha;
-            }
-            if (kFix) {
-                const bool wneed = __any(need);
-                if (lane == 0) flag_s[w] = wneed ? 1 : 0;
-            }
-            lds_barrier();                                   // Y: P(t), alpha, flags
-            if (kFix) {
-                const int4 fl = *reinterpret_cast<const int4 *>(flag_s);
-                if (fl.x | fl.y | fl.z | fl.w) {
-                    slow = true;
-                    break;
-                }
-            }
-            // ---- O += P . V ----
-            pv_step<kPrefillPLo>(phi, plo, lane, lds_addr(st) + va[0], lds_addr(st) + va[1], o);
-        }
-        if (kFix && slow) {
-            // a row's reference max moved: finish tile t with O rows rescaled
-            // (O passes through VGPRs; Q^T is dropped meanwhile and reloaded)
-#pragma unroll
-            for (int rt8 = 0; rt8 < 8; ++rt8) {
-                const float4_t al = *reinterpret_cast<const float4_t *>(&alpha_s[16 * rt8 + 4 * g]);
-#pragma unroll
-                for (int dt = 0; dt < 8; ++dt) o[rt8][dt] *= al;
-            }
-            const uint8_t *st = stages[t & 1];
-            pv_step<kPrefillPLo>(phi, plo, lane, lds_addr(st) + va[0], lds_addr(st) + va[1], o);
-            load_q(A, q_ok ? qi : 0, w, n16, g, qf);
-            ++t;
-        }
-    }
-
-    // ---- finish: l over the 4 key groups; publish m, l per row ----
-#pragma unroll
-    for (int rt = 0; rt < 2; ++rt) {
-        const float l = xsum_16_32(l_part[rt]);
-        if (g == 0) {
-            fin_s[0][32 * w + 16 * rt + n16] = m_use[rt];
-            fin_s[1][32 * w + 16 * rt + n16] = l;
-        }
-    }
-    if (!kFix) {
-        const bool wf = __any(failed);
-        if (lane == 0) flag_s[w] = wf ? 1 : 0;
-    }
-    lds_barrier();
-    if (!kFix) {
-        const int4 fl = *reinterpret_cast<const int4 *>(flag_s);
-        if (fl.x | fl.y | fl.z | fl.w) {
-            if (tid == 0) A.fail[pair] = 1;
-            return;
-        }
-    }
-#pragma unroll
-    for (int rt8 = 0; rt8 < 8; ++rt8) {
-        const int qq = q0 + (rt8 >> 2);
-        if (qq >= A.n_q) continue;
-        float inv[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int row = 16 * rt8 + 4 * g + r;
-            const int head = row & 63;
-            const float m = fin_s[0][row], l = fin_s[1][row];
-            const float sk = A.sinks[head] * kLog2e;
-            // the sink joins the denominator relative to the row's reference max
-            inv[r] = m == -INFINITY ? 0.0f : 1.0f / (l + __builtin_amdgcn_exp2f(sk - m));
-        }
-        float *dst = A.out + ((long long)qq * kH + ((16 * rt8) & 63) + 4 * g) * kD + 128 * w + n16;
-#pragma unroll
-        for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) dst[r * kD + 16 * dt] = o[rt8][dt][r] * inv[r];
     }
 }
 
@@ -478,12 +289,12 @@ __device__ inline void qk_tile(const uint8_t *st, const uint32_t *ka, const half
     asm volatile("s_nop 7\n\ts_nop 7" ::: "memory");
 }
 
-// Softmax of one tile with the reference max fixed (set on the first tile):
-// writes P hi/lo for the wave's two row tiles and accumulates l. A score more
-// than 2^kLazy above the reference marks the wave failed.
+// Softmax of one tile with the reference fixed (kFirst: set here, from this
+// tile): writes P hi/lo for the wave's two row tiles and accumulates l and the
+// largest growth over the reference.
 template <bool kFirst, bool kPLo>
 __device__ inline void softmax_fixed(const float4_t (*acc)[2], float kq_log2, int key0, int qpos,
-                                     int g, float *m_use, float *l_part, bool &failed,
+                                     int g, float *m_use, float *l_part, float *grow,
                                      half8_t *hi_out, half8_t *lo_out) {
     const bool edge = key0 + kTile - 1 > qpos;
 #pragma unroll
@@ -503,33 +314,51 @@ __device__ inline void softmax_fixed(const float4_t (*acc)[2], float kq_log2, in
         }
         const float m = m_use[rt];
         half8_t hi, lo;
-        float lsum = 0.0f;
-        bool big = false;
+        float lsum = 0.0f, gr = grow[rt];
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float x = s2[kt][r] - m;
-                big |= x > kLazy;
+                const float x = s2[kt][r] - m;   // NaN only where both are -inf (nothing visible yet)
+                gr = fmaxf(gr, x);
                 const float p = s2[kt][r] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(x);
                 const half_t h = (half_t)p;
                 lsum += kPLo ? p : (float)h;
                 hi[4 * kt + r] = h;
                 if (kPLo) lo[4 * kt + r] = (half_t)(p - (float)h);
             }
+        grow[rt] = gr;
         l_part[rt] += lsum;
-        failed |= big;
         hi_out[rt] = hi;
         lo_out[rt] = lo;
     }
 }
 
-// The fast kernel: software-pipelined over tiles with one barrier per tile.
+// The growth alone, of a pass whose P is not needed any more.
+__device__ inline void grow_only(const float4_t (*acc)[2], float kq_log2, int key0, int qpos, int g,
+                                 const float *m_use, float *grow) {
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (key0 + pi_key(16 * kt + 4 * g + r) <= qpos)
+                    grow[rt] = fmaxf(grow[rt], acc[kt][rt][r] * kq_log2 - m_use[rt]);
+}
+
+// One pass over a pair's tiles (or a part of them), software-pipelined with one
+// barrier per tile. kSecond: only the slots whose first pass outgrew its
+// reference, from their row maxima (so that no P exceeds 1) and with P as
+// hi + lo. A second pass costs what the first does; rescaling O where a
+// reference moves cost more (its 256 accumulators are AGPRs, which only MFMAs
+// operate on). Rows with 1% x8: 333 queries over 1001 506 -> 187 us, 20 over
+// 4000 1324 -> 71 us, 1024 over 1001 1480 -> 412 us.
 // Iteration t: [barrier] S(t) = K(t) Q^T | dequantize tile t+1 (fetched one
 // iteration earlier), fetch tile t+2 | softmax(t) | O += P(t-1) V(t-1). Three f16 stages (t-1 for V, t for K,
 // t+1 being written) and two P buffers make every LDS hazard one barrier apart.
-template <bool kPLo>
-__global__ __launch_bounds__(256) void prefill_fast_kernel(const PrefillArgs A) {
+template <bool kPLo, bool kSecond>
+__global__ __launch_bounds__(256) void prefill_kernel(const PrefillArgs A) {
     __shared__ __attribute__((aligned(16))) uint8_t stages[3][kStageB];
     __shared__ __attribute__((aligned(16))) half8_t pb[2][2][8][64];   // [buf][hi,lo][row tile][lane]
     __shared__ __attribute__((aligned(16))) int flag_s[4];
@@ -537,13 +366,26 @@ __global__ __launch_bounds__(256) void prefill_fast_kernel(const PrefillArgs A) 
 
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int n16 = lane & 15, g = lane >> 4;
-    const int pair = (int)gridDim.x - 1 - (int)blockIdx.x;
+    // the longest pairs first
+    const int slot = (int)gridDim.x - 1 - (int)blockIdx.x;
+    if (kSecond && A.fail[slot] == 0) return;
+    const int pair = slot / A.parts;
     const int q0 = 2 * pair;
     const int qi = q0 + (w >> 1);
     const bool q_ok = qi < A.n_q;
     const int qpos = q_ok ? A.n_cached + qi : -1;
     const int n_all = A.n_cached + (q0 + 2 < A.n_q ? q0 + 2 : A.n_q);
-    const int n_tiles = (n_all + kTile - 1) / kTile;
+    // this part's tiles [t0, t1)
+    const int all_tiles = (n_all + kTile - 1) / kTile, per = (all_tiles + A.parts - 1) / A.parts;
+    const int t0 = (slot % A.parts) * per, t1 = min(t0 + per, all_tiles);
+    if (t0 >= t1) {   // a short pair has fewer parts: an empty partial
+        if (tid < kRows) {
+            A.part_ml[(size_t)slot * 2 * kRows + tid] = -INFINITY;
+            A.part_ml[(size_t)slot * 2 * kRows + kRows + tid] = 0.0f;
+        }
+        if (tid == 0) A.fail[slot] = 0;
+        return;
+    }
 
     half8_t qf[2][16];
     load_q(A, q_ok ? qi : 0, w, n16, g, qf);
@@ -552,8 +394,10 @@ __global__ __launch_bounds__(256) void prefill_fast_kernel(const PrefillArgs A) 
     for (int a = 0; a < 8; ++a)
 #pragma unroll
         for (int b = 0; b < 8; ++b) o[a][b] = float4_t{0, 0, 0, 0};
-    float m_use[2], l_part[2] = {0.f, 0.f};
-    bool failed = false;
+    float m_use[2], l_part[2] = {0.f, 0.f}, grow[2] = {0.f, 0.f};
+    if (kSecond)
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt) m_use[rt] = A.row_max[(size_t)slot * kRows + 32 * w + 16 * rt + n16];
 
     uint32_t ka[2];
 #pragma unroll
@@ -569,17 +413,17 @@ __global__ __launch_bounds__(256) void prefill_fast_kernel(const PrefillArgs A) 
     }
 
     Raw R;
-    load_raw(A, 0, n_all, tid, R);
+    load_raw(A, t0, n_all, tid, R);
     store_tile(stages[0], tid, R);
-    load_raw(A, 1, n_all, tid, R);
+    load_raw(A, t0 + 1, n_all, tid, R);
     lds_barrier();
     {
         float4_t acc[2][2];
         qk_tile(stages[0], ka, qf, acc);
         store_tile(stages[1], tid, R);
-        load_raw(A, 2, n_all, tid, R);
+        load_raw(A, t0 + 2, n_all, tid, R);
         half8_t hi[2], lo[2];
-        softmax_fixed<true, kPLo>(acc, A.kq_log2, 0, qpos, g, m_use, l_part, failed, hi, lo);
+        softmax_fixed<!kSecond, kPLo>(acc, A.kq_log2, t0 * kTile, qpos, g, m_use, l_part, grow, hi, lo);
 #pragma unroll
         for (int rt = 0; rt < 2; ++rt) {
             pb[0][0][2 * w + rt][lane] = hi[rt];
@@ -587,50 +431,98 @@ __global__ __launch_bounds__(256) void prefill_fast_kernel(const PrefillArgs A) 
         }
     }
     int sp = 0, sc = 1, sn = 2;   // stages of tiles t-1, t, t+1
-    for (int t = 1; t < n_tiles; ++t) {
-        lds_barrier();
-        float4_t acc[2][2];
-        qk_tile(stages[sc], ka, qf, acc);
-        // tile t+1 (fetched one iteration ago) is dequantized; t+2 is fetched
-        store_tile(stages[sn], tid, R);
-        load_raw(A, t + 2, n_all, tid, R);
-        half8_t hi[2], lo[2];
-        softmax_fixed<false, kPLo>(acc, A.kq_log2, t * kTile, qpos, g, m_use, l_part, failed, hi, lo);
-        const int pbuf = (t - 1) & 1;
+    int pbuf = 0, t = t0 + 1;
+    bool stop = false;
+    if (!kSecond && tid == 0) flag_s[0] = 0;   // read after more barriers
+    // the reference is looked at every kCheckTiles tiles: inside the tile loop
+    // the check cost 3.5%. (A wave may see another's mark a round earlier than
+    // the rest; both loops have one barrier a tile, and the slot is redone.)
+    while (t < t1 && !stop) {
+        const int t_check = min(t + kCheckTiles, t1);
+        for (; t < t_check; ++t, pbuf ^= 1) {
+            lds_barrier();
+            float4_t acc[2][2];
+            qk_tile(stages[sc], ka, qf, acc);
+            // tile t+1 (fetched one iteration ago) is dequantized; t+2 is fetched
+            store_tile(stages[sn], tid, R);
+            load_raw(A, t + 2, n_all, tid, R);
+            half8_t hi[2], lo[2];
+            softmax_fixed<false, kPLo>(acc, A.kq_log2, t * kTile, qpos, g, m_use, l_part, grow, hi, lo);
 #pragma unroll
-        for (int rt = 0; rt < 2; ++rt) {
-            pb[pbuf ^ 1][0][2 * w + rt][lane] = hi[rt];
-            if (kPLo) pb[pbuf ^ 1][1][2 * w + rt][lane] = lo[rt];
+            for (int rt = 0; rt < 2; ++rt) {
+                pb[pbuf ^ 1][0][2 * w + rt][lane] = hi[rt];
+                if (kPLo) pb[pbuf ^ 1][1][2 * w + rt][lane] = lo[rt];
+            }
+            pv_step<kPLo>(pb[pbuf][0], pb[pbuf][1], lane, lds_addr(stages[sp]) + va[0],
+                    lds_addr(stages[sp]) + va[1], o);
+            const int tmp = sp;
+            sp = sc;
+            sc = sn;
+            sn = tmp;
         }
-        pv_step<kPLo>(pb[pbuf][0], pb[pbuf][1], lane, lds_addr(stages[sp]) + va[0],
-                lds_addr(stages[sp]) + va[1], o);
-        const int tmp = sp;
-        sp = sc;
-        sc = sn;
-        sn = tmp;
+        if (!kSecond) {
+            volatile int *mark = &flag_s[0];
+            if (__any(fmaxf(grow[0], grow[1]) > kLazy) && lane == 0) *mark = 1;
+            stop = __builtin_amdgcn_readfirstlane(*mark) != 0;
+        }
+    }
+    if (!kSecond && stop) {
+        // the second pass will redo this slot: only the rows' maxima are still
+        // needed (QK^T without P . V, a third of a tile's time)
+        for (; t < t1; ++t) {
+            lds_barrier();
+            float4_t acc[2][2];
+            qk_tile(stages[sc], ka, qf, acc);
+            store_tile(stages[sn], tid, R);
+            load_raw(A, t + 2, n_all, tid, R);
+            grow_only(acc, A.kq_log2, t * kTile, qpos, g, m_use, grow);
+            const int tmp = sp;
+            sp = sc;
+            sc = sn;
+            sn = tmp;
+        }
     }
     lds_barrier();
-    {
-        const int pbuf = (n_tiles - 1) & 1;
-        pv_step<kPLo>(pb[pbuf][0], pb[pbuf][1], lane, lds_addr(stages[sp]) + va[0],
-                lds_addr(stages[sp]) + va[1], o);
-    }
+    if (kSecond || !stop)
+        pv_step<kPLo>(pb[pbuf][0], pb[pbuf][1], lane, lds_addr(stages[sp]) + va[0], lds_addr(stages[sp]) + va[1], o);
 
     // ---- finish ----
+    bool failed = false;
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt) {
         const float l = xsum_16_32(l_part[rt]);
+        const float gr = xmax_16_32(grow[rt]);
+        failed |= gr > kLazy;
         if (g == 0) {
-            fin_s[0][32 * w + 16 * rt + n16] = m_use[rt];
-            fin_s[1][32 * w + 16 * rt + n16] = l;
+            const int row = 32 * w + 16 * rt + n16;
+            fin_s[0][row] = m_use[rt];
+            fin_s[1][row] = l;
+            if (!kSecond) A.row_max[(size_t)slot * kRows + row] = m_use[rt] + gr;
         }
     }
-    const bool wf = __any(failed);
-    if (lane == 0) flag_s[w] = wf ? 1 : 0;
+    if (!kSecond) {
+        const bool wf = __any(failed);
+        if (lane == 0) flag_s[w] = wf ? 1 : 0;
+    }
     lds_barrier();
-    const int4 fl = *reinterpret_cast<const int4 *>(flag_s);
-    if (fl.x | fl.y | fl.z | fl.w) {
-        if (tid == 0) A.fail[pair] = 1;
+    if (!kSecond) {
+        const int4 fl = *reinterpret_cast<const int4 *>(flag_s);
+        const bool fail = (fl.x | fl.y | fl.z | fl.w) != 0;
+        if (tid == 0) A.fail[slot] = fail ? 1 : 0;
+        if (fail) return;
+    }
+    if (A.parts > 1) {
+        if (tid < kRows) {
+            A.part_ml[(size_t)slot * 2 * kRows + tid] = fin_s[0][tid];
+            A.part_ml[(size_t)slot * 2 * kRows + kRows + tid] = fin_s[1][tid];
+        }
+        float *dst = A.part_o + ((size_t)slot * kRows + 4 * g) * kD + 128 * w + n16;
+#pragma unroll
+        for (int rt8 = 0; rt8 < 8; ++rt8)
+#pragma unroll
+            for (int dt = 0; dt < 8; ++dt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) dst[(16 * rt8 + r) * kD + 16 * dt] = o[rt8][dt][r];
         return;
     }
 #pragma unroll
@@ -643,6 +535,7 @@ __global__ __launch_bounds__(256) void prefill_fast_kernel(const PrefillArgs A) 
             const int row = 16 * rt8 + 4 * g + r;
             const float m = fin_s[0][row], l = fin_s[1][row];
             const float sk = A.sinks[row & 63] * kLog2e;
+            // the sink joins the denominator relative to the row's reference
             inv[r] = m == -INFINITY ? 0.0f : 1.0f / (l + __builtin_amdgcn_exp2f(sk - m));
         }
         float *dst = A.out + ((long long)qq * kH + ((16 * rt8) & 63) + 4 * g) * kD + 128 * w + n16;
@@ -653,15 +546,59 @@ __global__ __launch_bounds__(256) void prefill_fast_kernel(const PrefillArgs A) 
     }
 }
 
-__global__ void zero_i32_kernel(int *p, int n) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0;
+// The parts of a pair's keys and the sink, per row (query, head): one wave per
+// row half, a lane's four dims over the parts in order. Bound by the partials'
+// reads (2 KB a row and part).
+__global__ __launch_bounds__(256) void prefill_merge_kernel(const PrefillArgs A) {
+    const int lane = threadIdx.x & 63, unit = blockIdx.x * 4 + (threadIdx.x >> 6);   // row half
+    const int row = unit >> 1, qq = row / kH, head = row % kH;
+    if (qq >= A.n_q) return;
+    const int slot0 = (qq >> 1) * A.parts, r128 = (qq & 1) * kH + head;
+    const float *ml = A.part_ml + (size_t)slot0 * 2 * kRows + r128;
+    const float sink = A.sinks[head] * kLog2e;
+    float m = lane < A.parts ? ml[(size_t)lane * 2 * kRows] : -INFINITY;   // parts <= 64: one per lane
+    const float l = lane < A.parts ? ml[(size_t)lane * 2 * kRows + kRows] : 0.0f;
+    float mx = fmaxf(m, sink);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
+    const float sc = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mx);
+    float den = l * sc;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) den += __shfl_xor(den, off);
+    den += __builtin_amdgcn_exp2f(sink - mx);
+    const int d = (unit & 1) * (kD / 2) + 4 * lane;
+    const float *po = A.part_o + ((size_t)slot0 * kRows + r128) * kD + d;
+    float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 8
+    for (int i = 0; i < A.parts; ++i) {
+        const float c = __shfl(sc, i);
+        const float4_t o = *reinterpret_cast<const float4_t *>(po + (size_t)i * kRows * kD);
+        acc = c != 0.0f ? acc + o * c : acc;   // a select: an empty part's partial was never written
+    }
+    *reinterpret_cast<float4_t *>(A.out + ((size_t)qq * kH + head) * kD + d) = acc * (1.0f / den);
+}
+
+// Parts of every pair's keys: as many as fill kSplitWgs workgroups, of at
+// least kMinPartTiles tiles of the longest pair.
+int prefill_parts(int n_pairs, long long n_rows) {
+    const long long tiles = (n_rows + kTile - 1) / kTile;
+    const long long parts = std::min<long long>({kSplitWgs / n_pairs, tiles / kMinPartTiles, kMaxParts});
+    return (int)std::max<long long>(1, parts);
+}
+
+size_t up256(size_t b) { return (b + 255) & ~(size_t)255; }
+// fail flags and row maxima per slot, and with a split its partials
+size_t prefill_ws_bytes(size_t slots, bool split) {
+    size_t b = up256(slots * sizeof(int)) + up256(slots * kRows * sizeof(float));
+    if (split) b += up256(slots * 2 * kRows * sizeof(float)) + slots * kRows * kD * sizeof(float);
+    return b;
 }
 
 }  // namespace
 
 extern "C" size_t ds4hip_flash_attn_prefill_fp8_workspace_size(int n_q) {
-    return n_q > 0 ? (size_t)((n_q + 1) / 2) * sizeof(int) : 0;
+    // a split has at most kSplitWgs slots: enough for it and for one part a pair
+    return n_q > 0 ? std::max(prefill_ws_bytes(((size_t)n_q + 1) / 2, false), prefill_ws_bytes(kSplitWgs, true)) : 0;
 }
 
 extern "C" int ds4hip_flash_attn_prefill_fp8(const void *q, const float *sinks, float *out,
@@ -673,7 +610,7 @@ extern "C" int ds4hip_flash_attn_prefill_fp8(const void *q, const float *sinks, 
     if (n_head != kH || head_dim != kD || n_rot != kRot || n_q < 0 || n_cached < 0 ||
         (exact_p != 0 && exact_p != 1) ||
         (n_q > 0 && (!q || !sinks || !out || !codes || !sexp || !tail || !workspace ||
-                     workspace_bytes < ds4hip_flash_attn_prefill_fp8_workspace_size(n_q))))
+                     workspace_bytes < prefill_ws_bytes(((size_t)n_q + 1) / 2, false))))
         return ds4hip_set_last_error(kEINVAL);
     if (n_q == 0) return 0;
     const int n_pairs = (n_q + 1) / 2;
@@ -684,17 +621,28 @@ extern "C" int ds4hip_flash_attn_prefill_fp8(const void *q, const float *sinks, 
     A.codes = codes;
     A.sexp = sexp;
     A.tail = tail;
-    A.fail = static_cast<int *>(workspace);
+    A.parts = prefill_parts(n_pairs, (long long)n_cached + n_q);
+    if (workspace_bytes < prefill_ws_bytes((size_t)n_pairs * A.parts, A.parts > 1)) A.parts = 1;
+    const size_t slots = (size_t)n_pairs * A.parts;
+    char *c = static_cast<char *>(workspace);
+    A.fail = reinterpret_cast<int *>(c);
+    c += up256(slots * sizeof(int));
+    A.row_max = reinterpret_cast<float *>(c);
+    c += up256(slots * kRows * sizeof(float));
+    A.part_ml = reinterpret_cast<float *>(c);
+    c += up256(slots * 2 * kRows * sizeof(float));
+    A.part_o = reinterpret_cast<float *>(c);
     A.n_q = n_q;
     A.n_cached = n_cached;
     A.kq_log2 = kLog2e / sqrtf((float)kD);
     const hipStream_t st = (hipStream_t)stream;
-    hipLaunchKernelGGL(zero_i32_kernel, dim3((n_pairs + 255) / 256), dim3(256), 0, st, A.fail,
-                       n_pairs);
+    const dim3 grid((unsigned)slots);
     if (exact_p)
-        hipLaunchKernelGGL(prefill_fast_kernel<true>, dim3(n_pairs), dim3(256), 0, st, A);
+        hipLaunchKernelGGL((prefill_kernel<true, false>), grid, dim3(256), 0, st, A);
     else
-        hipLaunchKernelGGL(prefill_fast_kernel<false>, dim3(n_pairs), dim3(256), 0, st, A);
-    hipLaunchKernelGGL(prefill_fp8_kernel<true>, dim3(n_pairs), dim3(256), 0, st, A);
+        hipLaunchKernelGGL((prefill_kernel<false, false>), grid, dim3(256), 0, st, A);
+    hipLaunchKernelGGL((prefill_kernel<true, true>), grid, dim3(256), 0, st, A);
+    if (A.parts > 1)
+        hipLaunchKernelGGL(prefill_merge_kernel, dim3((unsigned)((long long)n_q * kH * 2 + 3) / 4), dim3(256), 0, st, A);
     return ds4hip_set_last_error(hip_status(hipGetLastError()));
 }

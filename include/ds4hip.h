@@ -234,9 +234,12 @@ long long ds4hip_flash_attn_q_prep_words(void);
  * own rows must already be in the cache (rows n_cached .. n_cached+n_q-1).
  * q [n_q][64][512] bf16 bits, sinks [64] fp32, out [n_q][64][512] fp32;
  * codes/sexp/tail point at the sequence's row 0. workspace holds
- * ds4hip_flash_attn_prefill_fp8_workspace_size(n_q) bytes (one flag per query
- * pair: pairs whose softmax range outgrows the fast kernel are redone by a
- * second, rescaling kernel in the same call). exact_p: 0 passes P to the P . V
+ * ds4hip_flash_attn_prefill_fp8_workspace_size(n_q) bytes, a size that also
+ * serves every smaller n_q (the partials of a small chunk, whose keys are split
+ * over workgroups; flags and row maxima of the query pairs whose softmax range
+ * outgrows the first pass, which a second one in the same call redoes). With
+ * less, down to 516 bytes per query pair and 512 more, the keys are not split.
+ * exact_p: 0 passes P to the P . V
  * MFMAs as one f16 (l sums the rounded values, so each output stays an exactly
  * normalized average), 1 as f16 hi + lo halves (~22 bits, twice the P . V
  * MFMAs). Per call; nothing is process-wide. */

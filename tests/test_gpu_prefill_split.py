@@ -1,0 +1,74 @@
+"""Prefill of small chunks (each pair's keys split over workgroups and merged)
+and of rows that outgrow the first pass's reference, against the oracle: the
+part counts' edges (one part, two, the most, pairs with fewer tiles than
+parts), odd query counts, and a row maximum in the last tile."""
+import numpy as np
+import pytest
+import torch
+
+from ds4cuda_amd import synth
+from test_gpu_decode import check, make_cache, q_bf16, sinks_for
+from test_gpu_prefill import oracle_prefill, run
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("outlier", [0.0, 0.02])
+@pytest.mark.parametrize("exact_p", [False, True])
+@pytest.mark.parametrize("n_cached,n_q", [(127, 1), (255, 1), (2100, 3), (8200, 2), (600, 31), (250, 255), (250, 258)])
+def test_prefill_split(gpu, n_cached, n_q, exact_p, outlier):
+    cache, (codes, sexp, tail) = make_cache(n_cached + n_q, 31 + n_q, gpu, outlier=outlier)
+    bits, qf = q_bf16(32, n_q)
+    sinks = sinks_for(33, 1)[0]
+    got = run(gpu, cache, bits, sinks, n_q, n_cached, exact_p=exact_p)
+    ref = oracle_prefill(qf, codes, sexp, tail, n_cached, sinks)
+    for t in range(n_q):
+        check(got[t], ref[t])
+
+
+@pytest.mark.parametrize("n_cached,n_q", [(1000, 2), (400, 270)])
+def test_prefill_late_maximum(gpu, n_cached, n_q):
+    # the last cached row draws all of query 0's attention: its score outgrows
+    # every reference by far more than the first pass allows
+    from ds4cuda_amd import ops
+    bits, qf = q_bf16(35, n_q)
+    x = synth.kv_rows(34, 0, n_cached + n_q)
+    x[n_cached - 1] = 6.0 * qf[0, 5]
+    cache = ops.Fp8KVCache.empty(n_cached + n_q, device=gpu)
+    cache.append(torch.from_numpy(x).to(gpu))
+    torch.cuda.synchronize()
+    codes, sexp = cache.codes.cpu().numpy(), cache.sexp.cpu().numpy()
+    tail = cache.tail.cpu().numpy().view(np.uint16)
+    sinks = sinks_for(36, 1)[0]
+    got = run(gpu, cache, bits, sinks, n_q, n_cached)
+    ref = oracle_prefill(qf, codes, sexp, tail, n_cached, sinks)
+    for t in range(n_q):
+        check(got[t], ref[t])
+
+
+def test_prefill_workspace_of_another_size(gpu):
+    """A workspace sized for a large chunk serves a small one (split), and one
+    with room for the flags alone runs it unsplit: the same outputs."""
+    import ctypes as C
+
+    from ds4cuda_amd._lib import lib
+    from ds4cuda_amd.ops import _ptr, _stream
+    n_cached, n_q = 900, 5
+    size = lib().ds4hip_flash_attn_prefill_fp8_workspace_size
+    assert all(size(a) <= size(b) for a, b in ((1, 2), (5, 300), (300, 511), (511, 513), (513, 4096)))
+    cache, (codes, sexp, tail) = make_cache(n_cached + n_q, 41, gpu)
+    bits, qf = q_bf16(42, n_q)
+    sinks = sinks_for(43, 1)[0]
+    ref = oracle_prefill(qf, codes, sexp, tail, n_cached, sinks)
+    q = torch.from_numpy(bits.view(np.int16)).to(gpu).view(torch.bfloat16)
+    s = torch.from_numpy(np.ascontiguousarray(sinks, np.float32)).to(gpu)
+    for nb, rc in ((size(4096), 0), (3 * 516 + 512, 0), (256, -22)):
+        out = torch.full((n_q, 64, 512), float("nan"), device=gpu)
+        ws = torch.empty(nb, dtype=torch.uint8, device=gpu)
+        assert lib().ds4hip_flash_attn_prefill_fp8(
+            _ptr(q), _ptr(s), _ptr(out), _ptr(cache.codes), _ptr(cache.sexp), _ptr(cache.tail), n_q, n_cached, 64, 512,
+            64, _ptr(ws), C.c_size_t(nb), 0, _stream(None)) == rc
+        torch.cuda.synchronize()
+        if rc == 0:
+            for t in range(n_q):
+                check(out[t].cpu().numpy(), ref[t])
