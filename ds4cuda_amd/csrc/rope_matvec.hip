@@ -73,6 +73,14 @@ __device__ inline float wave_sum(float v) {
     return v;
 }
 
+__device__ inline float block_sum_256(float v, float *part) {
+    v = wave_sum(v);
+    const int wave = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) part[wave] = v;
+    __syncthreads();
+    return ((part[0] + part[1]) + part[2]) + part[3];
+}
+
 // ---- f16 x fp32 matvec (cuda/router.cu:69-97) -----------------------------------------
 // 256 threads = 4 waves, 2 rows per wave; x staged in LDS as fp32.
 constexpr int kMvMaxIn = 16384;
@@ -314,6 +322,257 @@ __global__ __launch_bounds__(64 * 32 / kRpw) void mv_q8_quant_kernel(const uint8
     if (l == 0) yscale[blockIdx.x] = d;
 }
 
+// ---- the streamed form: rows of 32 or 128 blocks --------------------------------------------
+//
+// A row is read 68 bytes per lane (a pair of blocks), so a wave's loads straight
+// from memory touch every line of its rows 17 times: the matvec ran at 2.4 -
+// 4.2 TB/s, bound by the address unit. Here a wave copies 17408 consecutive
+// weight bytes (16 or 4 rows) to LDS with 17 copies of 1 KB each, all in
+// flight, and takes the pairs from there (17 dwords apart: no bank conflicts).
+// Two workgroups per CU hold 139 KB in flight, so a 35.7 MB matrix is one or
+// two waves' worth of copies per SIMD. Sums as in q8_rows: a lane's pairs in
+// order, then the butterfly (rows of 16 pairs use 16 lanes, whose butterfly
+// leaves out only the steps that would add zeros), so results are the same
+// bits. Measured (kernel alone): 32768 x 1024 with its norm and quantization
+// 19.6 us in two launches -> 9.9, the grouped 8 x 1024 x 4096 with its output's
+// quantization 10.3 -> 10.0 us. Rows of 256 blocks keep a wave per row (8192
+// columns x 4096 rows: 8.5 us against 8.9 streamed).
+constexpr int kStreamBytes = 17408, kStreamBlocks = kStreamBytes / 34;   // per wave: 512 blocks
+
+// Activations in LDS: pair p's 64 int8 at dword 17 p, then the block scales.
+template <int kNb>
+struct Q8X {
+    int q[kNb / 2 * 17];
+    float s[kNb];
+};
+
+// Issues the wave's copies; q8_stream_dot waits for them.
+__device__ inline void q8_stream_load(const uint8_t *w, uint8_t *lds, int lane) {
+#pragma unroll
+    for (int k = 0; k < kStreamBytes / 1024; ++k)
+        __builtin_amdgcn_global_load_lds(w + 1024 * k + 16 * lane, lds + 1024 * k, 16, 0, 0);
+}
+
+// One pair's two block terms added to acc (the even block first).
+__device__ inline float q8_pair(const uint32_t *d, const int *xb, float se, float so, float acc) {
+    uint32_t v[17], qe[8];
+    int x[16];
+#pragma unroll
+    for (int k = 0; k < 17; ++k) v[k] = d[k];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) x[k] = xb[k];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) qe[k] = __builtin_amdgcn_alignbyte(v[k + 1], v[k], 2);
+    acc += q8_block_term(f16_bits_to_f32((uint16_t)(v[0] & 0xFFFF)), se, qe, x);
+    acc += q8_block_term(f16_bits_to_f32((uint16_t)(v[8] >> 16)), so, v + 9, x + 8);
+    return acc;
+}
+
+// The wave's 512 / kNb row sums; put(row of the wave, sum) is called by one lane.
+template <int kNb, class F>
+__device__ inline void q8_stream_dot(const uint8_t *lds, const Q8X<kNb> &X, int lane, F put) {
+    constexpr int kPairs = kNb / 2, kRows = kStreamBlocks / kNb;
+    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): this wave's copies
+    asm volatile("" ::: "memory");
+    const uint32_t *w = reinterpret_cast<const uint32_t *>(lds);
+    if constexpr (kPairs == 16) {
+        const int g = lane >> 4, p = lane & 15;
+#pragma unroll
+        for (int i = 0; i < kRows / 4; ++i) {
+            const int r = 4 * i + g;
+            float a = q8_pair(w + (r * kPairs + p) * 17, X.q + 17 * p, X.s[2 * p], X.s[2 * p + 1], 0.0f);
+#pragma unroll
+            for (int off = 8; off > 0; off >>= 1) a += __shfl_xor(a, off);
+            if (p == 0) put(r, a);
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < kRows; ++r) {
+            float a = 0.0f;
+#pragma unroll
+            for (int u = 0; u < kPairs / 64; ++u) {
+                const int p = lane + 64 * u;
+                a = q8_pair(w + (r * kPairs + p) * 17, X.q + 17 * p, X.s[2 * p], X.s[2 * p + 1], a);
+            }
+            a = wave_sum(a);
+            if (lane == 0) put(r, a);
+        }
+    }
+}
+
+// The int8 value and scale of v in its 32-element block (the half-wave's 32
+// values): q8_quant_kernel's arithmetic.
+__device__ inline int q8_value(float v, float &d) {
+    float a = fabsf(v);
+#pragma unroll
+    for (int off = 16; off > 0; off >>= 1) a = fmaxf(a, __shfl_xor(a, off, 32));
+    d = a / 127.0f;
+    const float id = d != 0.0f ? 1.0f / d : 0.0f;
+    const int q = (int)__builtin_rintf(v * id);
+    return q > 127 ? 127 : (q < -128 ? -128 : q);
+}
+template <int kNb>
+__device__ inline void q8_put(Q8X<kNb> &X, int i, float v) {
+    float d;
+    const int q = q8_value(v, d);
+    reinterpret_cast<int8_t *>(X.q)[68 * (i >> 6) + (i & 63)] = (int8_t)q;
+    if ((i & 31) == 0) X.s[i >> 5] = d;
+}
+
+// Four consecutive elements of a 32-element block per lane (eight lanes a
+// block): the same values with three lane exchanges per block in place of five
+// per element; a maximum is the same in any order.
+template <int kNb>
+__device__ inline void q8_put4(Q8X<kNb> &X, int i, float4_t v) {
+    float a = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+    a = fmaxf(a, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), 0xB1, 0xF, 0xF, false)));
+    a = fmaxf(a, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), 0x4E, 0xF, 0xF, false)));
+    a = fmaxf(a, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), 0x141, 0xF, 0xF, false)));
+    const float d = a / 127.0f;
+    const float id = d != 0.0f ? 1.0f / d : 0.0f;
+    uint32_t q4 = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        int q = (int)__builtin_rintf(v[e] * id);
+        q = q > 127 ? 127 : (q < -128 ? -128 : q);
+        q4 |= ((uint32_t)q & 0xFFu) << (8 * e);
+    }
+    X.q[17 * (i >> 6) + ((i & 63) >> 2)] = (int)q4;
+    if ((i & 31) == 0) X.s[i >> 5] = d;
+}
+
+// What the activations are made of: int8 values and scales (kQ8), an fp32 row
+// quantized here (kF32), or an fp32 row normed and quantized here (kNorm:
+// norm_q8_kernel's arithmetic; workgroup 0 also writes the normed row).
+enum { kQ8 = 0, kF32 = 1, kNorm = 2 };
+struct Q8StreamArgs {
+    const uint8_t *w[2];      // [rows[0]] and [rows[1]] rows over the same input
+    float *y[2];
+    int rows[2];
+    const int8_t *xq;         // kQ8: [groups][32 kNb]; row r reads group r / rank
+    const float *xs;
+    int rank;
+    const float *x, *norm_w;  // kF32, kNorm
+    float *x_normed;
+    float eps;
+    int8_t *yq;               // kQuantOut: the rows' Q8_0 form in place of y[0]
+    float *yscale;
+};
+
+// kWaves waves of 512 / kNb rows each. kQuantOut: a workgroup's rows are whole
+// 32-row blocks, quantized as q8_quant_kernel would.
+template <int kNb, int kWaves, int kIn, bool kQuantOut>
+__global__ __launch_bounds__(64 * kWaves) void mv_q8_stream_kernel(const Q8StreamArgs A) {
+    constexpr int kRows = kStreamBlocks / kNb, kN = 32 * kNb, kThreads = 64 * kWaves;
+    __shared__ __attribute__((aligned(16))) uint8_t w_s[kWaves][kStreamBytes];
+    __shared__ Q8X<kNb> X;
+    __shared__ float part[4], y_s[kQuantOut ? kRows * kWaves : 1];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), tid = threadIdx.x;
+    const int blk_row = (int)blockIdx.x * kRows * kWaves;
+    const bool second = blk_row >= A.rows[0];
+    const int row0 = blk_row - (second ? A.rows[0] : 0) + wave * kRows;
+    // (a wave past the matrix's last rows has nothing to copy; its barriers stay)
+    const bool live = row0 < A.rows[second ? 1 : 0];
+    if constexpr (kIn == kQ8) {
+        // the first matrix only: 16 bytes a thread, written as dwords (pairs sit 17 dwords apart)
+        const int group = blk_row / A.rank;
+        const uint4_t *src = reinterpret_cast<const uint4_t *>(A.xq + (size_t)group * kN);
+        constexpr int kChunks = kN / 16, kPer = (kChunks + kThreads - 1) / kThreads;
+        uint4_t v[kPer];
+        float sv = 0.0f;
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) v[k] = src[min(tid + kThreads * k, kChunks - 1)];
+        if (tid < kNb) sv = A.xs[(size_t)group * kNb + tid];
+        if (live) q8_stream_load(A.w[0] + (size_t)row0 * kNb * 34, w_s[wave], lane);
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) {
+            const int c = tid + kThreads * k;
+            if (c < kChunks)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) X.q[17 * (c >> 2) + 4 * (c & 3) + e] = (int)v[k][e];
+        }
+        if (tid < kNb) X.s[tid] = sv;
+    } else {
+        constexpr int kPer = kN / kThreads;
+        const uint8_t *wrow = A.w[second ? 1 : 0] + (size_t)row0 * kNb * 34;
+        if constexpr (kIn == kF32) {
+            float4_t v[kPer / 4];
+            const bool wide = (reinterpret_cast<uintptr_t>(A.x) & 15) == 0;
+#pragma unroll
+            for (int k = 0; k < kPer / 4; ++k) {
+                const float *p = A.x + 4 * (tid + kThreads * k);
+                v[k] = wide ? *reinterpret_cast<const float4_t *>(p) : float4_t{p[0], p[1], p[2], p[3]};
+            }
+            if (live) q8_stream_load(wrow, w_s[wave], lane);
+#pragma unroll
+            for (int k = 0; k < kPer / 4; ++k) q8_put4(X, 4 * (tid + kThreads * k), v[k]);
+        } else {
+            static_assert(kThreads == 256, "the norm's sum order");
+            float v[kPer], nw[kPer], ss = 0.0f;
+#pragma unroll
+            for (int k = 0; k < kPer; ++k) v[k] = A.x[tid + kThreads * k];
+#pragma unroll
+            for (int k = 0; k < kPer; ++k) nw[k] = A.norm_w[tid + kThreads * k];
+            if (live) q8_stream_load(wrow, w_s[wave], lane);
+#pragma unroll
+            for (int k = 0; k < kPer; ++k) ss = fmaf(v[k], v[k], ss);
+            const float scale = 1.0f / sqrtf(block_sum_256(ss, part) / (float)kN + A.eps);
+#pragma unroll
+            for (int k = 0; k < kPer; ++k) {
+                v[k] = v[k] * scale * nw[k];
+                if (blockIdx.x == 0) A.x_normed[tid + kThreads * k] = v[k];
+                q8_put(X, tid + kThreads * k, v[k]);
+            }
+        }
+    }
+    __syncthreads();
+    if (live)
+        q8_stream_dot<kNb>(w_s[wave], X, lane, [&](int r, float v) {
+            if constexpr (kQuantOut) y_s[wave * kRows + r] = v;
+            else A.y[second ? 1 : 0][row0 + r] = v;
+        });
+    if constexpr (kQuantOut) {
+        static_assert(kRows * kWaves % 32 == 0, "whole Q8_0 blocks per workgroup");
+        __syncthreads();
+        if (tid < kRows * kWaves) {
+            float d;
+            A.yq[blk_row + tid] = (int8_t)q8_value(y_s[tid], d);
+            if ((tid & 31) == 0) A.yscale[(blk_row + tid) / 32] = d;
+        }
+    }
+}
+
+// Whether mv_q8_stream_kernel<n_blocks, waves> takes a matrix: whole waves of
+// rows, and copies of 16-byte aligned weights and activations.
+bool q8_stream_ok(const void *W, const void *xq, int n_rows, int n_blocks) {
+    return (n_blocks == 32 || n_blocks == 128) && n_rows % (kStreamBlocks / n_blocks) == 0 &&
+           ((reinterpret_cast<uintptr_t>(W) | reinterpret_cast<uintptr_t>(xq)) & 15) == 0;
+}
+
+// Q8_0 matvec of quantized activations (one group): the streamed form where it
+// applies, else one wave per row.
+void launch_mv_q8(const uint8_t *W, const int8_t *xq, const float *xs, float *y, int n_rows, int n_blocks, int rank,
+                  bool grouped, hipStream_t st) {
+    constexpr int kWaves = 4;
+    const int wg_rows = n_blocks > 0 && n_blocks <= kStreamBlocks ? kWaves * (kStreamBlocks / n_blocks) : 0;
+    // (a workgroup's rows read one group's activations)
+    if (q8_stream_ok(W, xq, n_rows, n_blocks) && (!grouped || rank % wg_rows == 0)) {
+        Q8StreamArgs A{};
+        A.w[0] = W;
+        A.y[0] = y;
+        A.rows[0] = n_rows;
+        A.xq = xq;
+        A.xs = xs;
+        A.rank = grouped ? rank : n_rows;
+        const dim3 g((n_rows + wg_rows - 1) / wg_rows), b(64 * kWaves);
+        if (n_blocks == 32) hipLaunchKernelGGL((mv_q8_stream_kernel<32, kWaves, kQ8, false>), g, b, 0, st, A);
+        else hipLaunchKernelGGL((mv_q8_stream_kernel<128, kWaves, kQ8, false>), g, b, 0, st, A);
+        return;
+    }
+    hipLaunchKernelGGL(mv_q8_kernel, dim3((n_rows + 3) / 4), dim3(256), 0, st, W, xq, xs, y, n_rows, n_blocks, rank,
+                       grouped ? 1 : 0);
+}
+
 // Steps 14 + 15a in one launch: the inverse tail RoPE of a head's attention
 // output and the Q8_0 quantization of the rotated row (one workgroup per
 // head, thread t on dims 2t and 2t + 1; a 32-dim block is 16 threads). The
@@ -353,8 +612,7 @@ int launch_q8(const uint8_t *W, const float *x, float *y, int n_groups, int grou
     int e = hip_status(hipGetLastError());
     if (e) return e;
     const int n_rows = grouped ? n_groups * rank : rank;
-    hipLaunchKernelGGL(mv_q8_kernel, dim3((n_rows + 3) / 4), dim3(256), 0, st, W, xq, xs, y,
-                       n_rows, bpg, rank, grouped ? 1 : 0);
+    launch_mv_q8(W, xq, xs, y, n_rows, bpg, rank, grouped, st);
     return hip_status(hipGetLastError());
 }
 
@@ -364,14 +622,6 @@ int launch_q8(const uint8_t *W, const float *x, float *y, int n_groups, int grou
 // wave sums are added in wave order, scale = 1 / sqrtf(ss / n + eps) and
 // y = x * scale * w (w NULL: unit gain), the reference's operation order.
 constexpr float kRmsEps = 1.0e-6f;
-
-__device__ inline float block_sum_256(float v, float *part) {
-    v = wave_sum(v);
-    const int wave = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) part[wave] = v;
-    __syncthreads();
-    return ((part[0] + part[1]) + part[2]) + part[3];
-}
 
 __global__ __launch_bounds__(256) void rms_norm_kernel(const float *__restrict__ x,
                                                        const float *__restrict__ w, int weight_dim,
@@ -413,20 +663,33 @@ __global__ __launch_bounds__(256) void norm_q8_kernel(const float *__restrict__ 
     }
 }
 
-// Per-head RMSNorm over 512 dims (optional weight shared by the heads), then
-// the tail RoPE of dims 448..511: one wave per head, lane l holds dims
-// 8 l .. 8 l + 7 (so lanes 56..63 hold the 32 rotated pairs, 4 each).
+// RMSNorm over 512 dims, then the tail RoPE of dims 448..511, of rows
+// [0, n_heads) of x (unit gain) and of one more row x2 (weight w2): one wave
+// per row, lane l holds dims 8 l .. 8 l + 7, so lanes 56..63 hold the 32
+// rotated pairs, 4 each. Lane t < 32 forms pair t's coefficients under the
+// row's loads, and those lanes fetch theirs (forming all four themselves, one
+// after the other, cost 2 us of the launch).
 __global__ __launch_bounds__(64) void head_norm_rope_kernel(const float *__restrict__ x,
                                                             const float *__restrict__ w,
-                                                            float *__restrict__ y, int pos,
+                                                            float *__restrict__ y, int n_heads,
+                                                            const float *__restrict__ x2,
+                                                            const float *__restrict__ w2,
+                                                            float *__restrict__ y2, int pos,
                                                             RopeParams P, float eps) {
     constexpr int kHd = 512, kNope = 448;
     const int l = threadIdx.x;
-    const float *xr = x + (size_t)blockIdx.x * kHd + 8 * l;
-    float *yr = y + (size_t)blockIdx.x * kHd + 8 * l;
-    float v[8];
+    const bool extra = (int)blockIdx.x >= n_heads;
+    const float *xr = (extra ? x2 : x + (size_t)blockIdx.x * kHd) + 8 * l;
+    float *yr = (extra ? y2 : y + (size_t)blockIdx.x * kHd) + 8 * l;
+    const float *wr = extra ? w2 : w;
+    float v[8], wv[8];
     const float4_t a = *reinterpret_cast<const float4_t *>(xr);
     const float4_t b = *reinterpret_cast<const float4_t *>(xr + 4);
+    if (wr)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) wv[i] = wr[8 * l + i];
+    float c, s;
+    rope_cs(l & 31, pos, P, c, s);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         v[i] = a[i];
@@ -437,11 +700,12 @@ __global__ __launch_bounds__(64) void head_norm_rope_kernel(const float *__restr
     for (int i = 0; i < 8; ++i) ss = fmaf(v[i], v[i], ss);
     const float scale = 1.0f / sqrtf(wave_sum(ss) / (float)kHd + eps);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = w ? v[i] * scale * w[8 * l + i] : v[i] * scale;
-    if (8 * l >= kNope) {
+    for (int i = 0; i < 8; ++i) v[i] = wr ? v[i] * scale * wv[i] : v[i] * scale;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            rope_pair(v[2 * i], v[2 * i + 1], (8 * l - kNope) / 2 + i, pos, P, v[2 * i], v[2 * i + 1]);
+    for (int i = 0; i < 4; ++i) {
+        const int t = ((8 * l - kNope) / 2 + i) & 31;   // the lane's pair, lanes 56..63
+        const float ct = __shfl(c, t), st = __shfl(s, t);
+        if (8 * l >= kNope) rope_apply(v[2 * i], v[2 * i + 1], ct, st, v[2 * i], v[2 * i + 1]);
     }
     *reinterpret_cast<float4_t *>(yr) = float4_t{v[0], v[1], v[2], v[3]};
     *reinterpret_cast<float4_t *>(yr + 4) = float4_t{v[4], v[5], v[6], v[7]};
@@ -905,10 +1169,22 @@ void attn_out_projections(const int8_t *xq, const float *xs, const void *w_out_a
                           hipStream_t st) {
     const int bpg = (n_head * head_dim) / n_groups / 32;
     const int n_low = n_groups * rank;
-    hipLaunchKernelGGL(mv_q8_quant_kernel<kQuantRpw>, dim3(n_low / 32), dim3(64 * 32 / kQuantRpw), 0, st,
-                       static_cast<const uint8_t *>(w_out_a), xq, xs, w.xq2, w.xs2, bpg, rank, 1);
-    hipLaunchKernelGGL(mv_q8_kernel, dim3((out_dim + 3) / 4), dim3(256), 0, st, static_cast<const uint8_t *>(w_out_b),
-                       w.xq2, w.xs2, out, out_dim, n_low / 32, out_dim, 0);
+    const uint8_t *wa = static_cast<const uint8_t *>(w_out_a);
+    if (bpg == 128 && q8_stream_ok(wa, xq, n_low, bpg)) {   // eight waves of four rows: one Q8_0 block
+        Q8StreamArgs A{};
+        A.w[0] = wa;
+        A.rows[0] = n_low;
+        A.xq = xq;
+        A.xs = xs;
+        A.rank = rank;
+        A.yq = w.xq2;
+        A.yscale = w.xs2;
+        hipLaunchKernelGGL((mv_q8_stream_kernel<128, 8, kQ8, true>), dim3(n_low / 32), dim3(512), 0, st, A);
+    } else {
+        hipLaunchKernelGGL(mv_q8_quant_kernel<kQuantRpw>, dim3(n_low / 32), dim3(64 * 32 / kQuantRpw), 0, st, wa, xq, xs,
+                           w.xq2, w.xs2, bpg, rank, 1);
+    }
+    launch_mv_q8(static_cast<const uint8_t *>(w_out_b), w.xq2, w.xs2, out, out_dim, n_low / 32, out_dim, false, st);
 }
 }  // namespace
 
@@ -1124,6 +1400,36 @@ extern "C" int ds4hip_attn_qkv_decode_f32(const float *attn_norm, const void *w_
     const uint8_t *qa = static_cast<const uint8_t *>(w_q_a);
     const uint8_t *kva = static_cast<const uint8_t *>(w_kv_a);
     const uint8_t *qb = static_cast<const uint8_t *>(w_q_b);
+    const RopeParams P = rope_params(64, il, false);
+    if (((reinterpret_cast<uintptr_t>(qa) | reinterpret_cast<uintptr_t>(kva) | reinterpret_cast<uintptr_t>(qb)) & 15) == 0) {
+        // three launches: q_a and kv_a, which quantize attn_norm themselves
+        // (Steps 3, 5); q_b, which norms and quantizes q_lora (Steps 4, 7);
+        // the norms and RoPEs of the 64 heads and of KV (Steps 6, 8 - 10).
+        // Seven launches took 42 us of kernels, these 20 us.
+        Q8StreamArgs A{};
+        A.w[0] = qa;
+        A.w[1] = kva;
+        A.y[0] = W.q_lora;
+        A.y[1] = W.kv_raw;
+        A.rows[0] = kQLora;
+        A.rows[1] = kKvDim;
+        A.x = attn_norm;
+        hipLaunchKernelGGL((mv_q8_stream_kernel<kEmbd / 32, 2, kF32, false>), dim3((kQLora + kKvDim) / 8), dim3(128), 0,
+                           st, A);
+        Q8StreamArgs B{};
+        B.w[0] = qb;
+        B.y[0] = W.q_raw;
+        B.rows[0] = kQDim;
+        B.x = W.q_lora;
+        B.norm_w = w_q_a_norm;
+        B.x_normed = q_lora_norm;
+        B.eps = kRmsEps;
+        hipLaunchKernelGGL((mv_q8_stream_kernel<kQLora / 32, 4, kNorm, false>), dim3(kQDim / 64), dim3(256), 0, st, B);
+        hipLaunchKernelGGL(head_norm_rope_kernel, dim3(65), dim3(64), 0, st, W.q_raw, nullptr, q_cur, 64, W.kv_raw,
+                           w_kv_a_norm, kv_rope, pos, P, kRmsEps);
+        return ds4hip_set_last_error(hip_status(hipGetLastError()));
+    }
+    // weights that are not 16-byte aligned: one launch per step
     // Steps 3 and 5: q_lora and KVraw from one quantization of attn_norm
     hipLaunchKernelGGL(q8_quant_kernel, dim3(kEmbd / 256), dim3(256), 0, st, attn_norm, W.xq, W.xs,
                        kEmbd / 32);
@@ -1134,13 +1440,10 @@ extern "C" int ds4hip_attn_qkv_decode_f32(const float *attn_norm, const void *w_
     // Step 4 with the quantization of Step 7's input; Steps 6 + 10
     hipLaunchKernelGGL(norm_q8_kernel, dim3(1), dim3(256), 0, st, W.q_lora, w_q_a_norm, q_lora_norm,
                        W.xq2, W.xs2, kQLora, kRmsEps);
-    const RopeParams P = rope_params(64, il, false);
-    hipLaunchKernelGGL(head_norm_rope_kernel, dim3(1), dim3(64), 0, st, W.kv_raw, w_kv_a_norm,
-                       kv_rope, pos, P, kRmsEps);
     // Step 7, then Steps 8 + 9
     hipLaunchKernelGGL(mv_q8_kernel, dim3(kQDim / 4), dim3(256), 0, st, qb, W.xq2, W.xs2, W.q_raw,
                        kQDim, kQLora / 32, kQDim, 0);
-    hipLaunchKernelGGL(head_norm_rope_kernel, dim3(64), dim3(64), 0, st, W.q_raw, nullptr, q_cur,
-                       pos, P, kRmsEps);
+    hipLaunchKernelGGL(head_norm_rope_kernel, dim3(65), dim3(64), 0, st, W.q_raw, nullptr, q_cur, 64, W.kv_raw,
+                       w_kv_a_norm, kv_rope, pos, P, kRmsEps);
     return ds4hip_set_last_error(hip_status(hipGetLastError()));
 }
