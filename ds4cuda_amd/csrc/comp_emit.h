@@ -72,24 +72,30 @@ __device__ inline void emit_row(const Src &src, const float *__restrict__ w_norm
                 v = den > 0.0f ? sum / den : 0.0f;
             }
         } else {
-            // ratio 128: the column's scores in registers and the values 32
-            // at a time, so that the loads of a batch are in flight together
-            // (row by row, an emit took 32 us with the state in cache; now 12)
-            float s[128];
+            // ratio 128: 32 rows at a time, so that the loads of a batch are in
+            // flight together (row by row, an emit took 32 us with the state in
+            // cache; now 12)
+#pragma unroll 1
+            for (int b = 0; b < 128; b += 32) {
+                float sc[32];
 #pragma unroll
-            for (int r = 0; r < 128; ++r) s[r] = src.score(r, j);
+                for (int r = 0; r < 32; ++r) sc[r] = src.score(b + r, j);
 #pragma unroll
-            for (int r = 0; r < 128; ++r) mx = fmaxf(mx, s[r]);
+                for (int r = 0; r < 32; ++r) mx = fmaxf(mx, sc[r]);
+            }
             if (mx > kNegInf * 0.5f) {
                 float den = 0.0f, sum = 0.0f;
-#pragma unroll
+#pragma unroll 1
                 for (int b = 0; b < 128; b += 32) {
-                    float k[32];
-#pragma unroll
-                    for (int r = 0; r < 32; ++r) k[r] = src.kv(b + r, j);
+                    float sc[32], k[32];
 #pragma unroll
                     for (int r = 0; r < 32; ++r) {
-                        const float w = expf(s[b + r] - mx);
+                        sc[r] = src.score(b + r, j);
+                        k[r] = src.kv(b + r, j);
+                    }
+#pragma unroll
+                    for (int r = 0; r < 32; ++r) {
+                        const float w = expf(sc[r] - mx);
                         den += w;
                         sum += w * k[r];
                     }

@@ -54,6 +54,7 @@ constexpr int kVtStride = 40;    // halves per V^T line (32 rows + 8 pad)
 constexpr int kMaxProb = 128;
 constexpr int kMinChunk = 2 * kTile;       // the register-load kernels run tiles in pairs
 constexpr int kMinChunkFlat = kTile;       // the flat-stage kernel: one tile is a whole chunk
+constexpr int kMinChunkF32 = kTile;        // and the fp32-row kernel
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLazyLog2 = 8.0f;   // decode softmax: reference point slack (log2 units)
 constexpr int kFp8WgPerCu = 1;   // the FP8 kernel's LDS ring allows one workgroup per CU
@@ -123,8 +124,20 @@ __device__ inline MergeRope merge_rope(const DecodeArgs &A, int p, int dim0) {
     constexpr int kNope = kD - kRot;
     if (A.out_form && dim0 >= kNope) {
         const int pos = A.rope_pos_dev ? A.rope_pos_dev[p] : A.rope_pos;
-        rope_cs((dim0 - kNope) / 2, pos, A.rope, r.c[0], r.s[0]);
-        rope_cs((dim0 + 2 - kNope) / 2, pos, A.rope, r.c[1], r.s[1]);
+        // one copy of the sine and cosine code (see the merges)
+        float cs[2][2];
+#pragma unroll 1
+        for (int i = 0; i < 2; ++i) {
+            rope_cs((dim0 - kNope) / 2 + i, pos, A.rope, cs[1][0], cs[1][1]);
+            if (i == 0) {
+                cs[0][0] = cs[1][0];
+                cs[0][1] = cs[1][1];
+            }
+        }
+        r.c[0] = cs[0][0];
+        r.s[0] = cs[0][1];
+        r.c[1] = cs[1][0];
+        r.s[1] = cs[1][1];
     }
     // here, not sunk next to their use at the end
     asm volatile("" : "+v"(r.c[0]), "+v"(r.c[1]), "+v"(r.s[0]), "+v"(r.s[1]));
@@ -257,61 +270,39 @@ __device__ inline void mark_slot(const DecodeArgs &A, long long slot, int p, int
     }
 }
 
-// fp32 rows (reference launchers): the lane's 16-dim slice of block b,
-// f16-rounded exactly like f16_round (cuda/flash_attn.cu:113-115).
-__device__ inline void load_f32_block(const float *row, int b, int q, bool valid,
-                                      half8_t &a0, half8_t &a1) {
-    if (!valid) {
-        a0 = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
-        a1 = a0;
-        return;
-    }
+// fp32 rows (reference launchers): the lane's 16-dim slice of block b, raw
+// (16 floats) and f16-rounded exactly like f16_round (cuda/flash_attn.cu:113-115),
+// zero for a row that takes no part.
+__device__ inline void load_f32_raw(const float *row, int b, int q, float4_t (&f)[4]) {
     const float4_t *p = reinterpret_cast<const float4_t *>(row + 64 * b + 16 * q);
-    a0 = f32x8_to_half8(p[0], p[1]);
-    a1 = f32x8_to_half8(p[2], p[3]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) f[i] = p[i];
+}
+__device__ inline void round_f32_block(const float4_t (&f)[4], bool valid, half8_t &a0, half8_t &a1) {
+    const half8_t z = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+    a0 = valid ? f32x8_to_half8(f[0], f[1]) : z;
+    a1 = valid ? f32x8_to_half8(f[2], f[3]) : z;
 }
 
-// Q^T B fragments of one problem: k-step 2b+s covers dims 64b+16q+8s+[0,8).
-template <bool kQf32>
-__device__ inline void load_q(const DecodeArgs &A, int p, int head, int q, half8_t *qh,
-                              half8_t *ql) {
-    if (kQf32) {
-        const float *src = static_cast<const float *>(A.q) + (long long)p * A.q_stride +
-                           (long long)head * kD + 16 * q;
+// Q^T B fragments (f16 hi and lo) of one problem's fp32 Q: k-step 2b+s covers
+// dims 64b+16q+8s+[0,8).
+__device__ inline void load_q(const DecodeArgs &A, int p, int head, int q, half8_t *qh, half8_t *ql) {
+    const float *src = static_cast<const float *>(A.q) + (long long)p * A.q_stride + (long long)head * kD;
 #pragma unroll
-        for (int b = 0; b < 8; ++b) {
+    for (int b = 0; b < 8; ++b) {
+        float4_t x[4];
+        load_f32_raw(src, b, q, x);
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                const float4_t x0 = *reinterpret_cast<const float4_t *>(src + 64 * b + 8 * s);
-                const float4_t x1 = *reinterpret_cast<const float4_t *>(src + 64 * b + 8 * s + 4);
-                half8_t hi, lo;
+        for (int s = 0; s < 2; ++s) {
+            half8_t hi, lo;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    hi[i] = (half_t)x0[i];
-                    lo[i] = (half_t)(x0[i] - (float)hi[i]);
-                    hi[4 + i] = (half_t)x1[i];
-                    lo[4 + i] = (half_t)(x1[i] - (float)hi[4 + i]);
-                }
-                qh[2 * b + s] = hi;
-                ql[2 * b + s] = lo;
+            for (int i = 0; i < 8; ++i) {
+                const float v = x[2 * s + (i >> 2)][i & 3];
+                hi[i] = (half_t)v;
+                lo[i] = (half_t)(v - (float)hi[i]);
             }
-        }
-    } else {
-        const uint16_t *src = static_cast<const uint16_t *>(A.q) + (long long)p * A.q_stride +
-                              (long long)head * kD + 16 * q;
-#pragma unroll
-        for (int b = 0; b < 8; ++b) {
-#pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                const uint4_t v = *reinterpret_cast<const uint4_t *>(src + 64 * b + 8 * s);
-                half8_t h;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    h[2 * i] = (half_t)bf16_to_f32((uint16_t)(v[i] & 0xFFFF));
-                    h[2 * i + 1] = (half_t)bf16_to_f32((uint16_t)(v[i] >> 16));
-                }
-                qh[2 * b + s] = h;
-            }
+            qh[2 * b + s] = hi;
+            ql[2 * b + s] = lo;
         }
     }
 }
@@ -357,17 +348,18 @@ __device__ inline void lds_barrier() {
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
+template <int kN>   // 16-dim column tiles of O
 struct SegState {
     float m_run;
     float l_run;
-    float4_t o[32];
+    float4_t o[kN];
 };
 
 // Online softmax of one 32-row tile (S^T accumulators acc[t][r] = row
 // 16t+4q+r, head j) and the P fragment for P . V. row_ok(t, r) says whether
 // that row takes part.
-template <typename RowOk>
-__device__ inline half8_t softmax_tile(const float4_t *acc, float kq_log2, int q, SegState &S,
+template <int kN, typename RowOk>
+__device__ inline half8_t softmax_tile(const float4_t *acc, float kq_log2, int q, SegState<kN> &S,
                                        RowOk row_ok) {
     float s[2][4];
     float tmax = -INFINITY;
@@ -401,16 +393,17 @@ __device__ inline half8_t softmax_tile(const float4_t *acc, float kq_log2, int q
 #pragma unroll
         for (int r = 0; r < 4; ++r) ar[r] = __shfl(alpha, 4 * q + r);
 #pragma unroll
-        for (int n = 0; n < 32; ++n)
+        for (int n = 0; n < kN; ++n)
 #pragma unroll
             for (int r = 0; r < 4; ++r) S.o[n][r] *= ar[r];
     }
     return pf;
 }
 
-__device__ inline void pv_tile(const half_t *vt, half8_t pf, int j, int q, SegState &S) {
+template <int kN>
+__device__ inline void pv_tile(const half_t *vt, half8_t pf, int j, int q, SegState<kN> &S) {
 #pragma unroll
-    for (int n = 0; n < 32; ++n) {
+    for (int n = 0; n < kN; ++n) {
         const half8_t vb = *reinterpret_cast<const half8_t *>(&vt[(16 * n + j) * kVtStride + 8 * q]);
         S.o[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pf, vb, S.o[n], 0, 0, 0);
     }
@@ -426,18 +419,22 @@ __device__ inline void vt_write(half_t *vt, int b, int q, int prow, half8_t a0, 
     }
 }
 
+// dim0: the first of the workgroup's dims; the first workgroup of a slot's
+// dims writes the scalars.
+template <int kN>
 __device__ inline void emit_partial(const DecodeArgs &A, long long slot, int wave, int j, int q,
-                                    int head, int p, SegState &S) {
+                                    int head, int p, int dim0, SegState<kN> &S) {
     float l = S.l_run;
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
-    float *wo = A.ws_o + slot * (kH * kD) + (wave * 16 + 4 * q) * kD + j;
-    // keep the 128 store addresses from being hoisted out of the tile loop
+    float *wo = A.ws_o + slot * (kH * kD) + (wave * 16 + 4 * q) * kD + dim0 + j;
+    // keep the store addresses from being hoisted out of the tile loop
     asm volatile("" : "+v"(wo));
 #pragma unroll
-    for (int n = 0; n < 32; ++n)
+    for (int n = 0; n < kN; ++n)
 #pragma unroll
         for (int r = 0; r < 4; ++r) wo[r * kD + 16 * n] = S.o[n][r];
+    if (dim0) return;
     if (q == 0) {
         A.ws_ml[slot * 2 * kH + head] = S.m_run;
         A.ws_ml[slot * 2 * kH + kH + head] = l;
@@ -445,11 +442,12 @@ __device__ inline void emit_partial(const DecodeArgs &A, long long slot, int wav
     if (threadIdx.x == 0) A.ws_prob[slot] = p;
 }
 
-__device__ inline void seg_init(SegState &S) {
+template <int kN>
+__device__ inline void seg_init(SegState<kN> &S) {
     S.m_run = -INFINITY;
     S.l_run = 0.0f;
 #pragma unroll
-    for (int n = 0; n < 32; ++n) S.o[n] = float4_t{0, 0, 0, 0};
+    for (int n = 0; n < kN; ++n) S.o[n] = float4_t{0, 0, 0, 0};
 }
 
 // ---- FP8 cache kernel ------------------------------------------------------------------
@@ -994,11 +992,20 @@ __global__ __launch_bounds__(256) void decode_fp8_kernel(const DecodeArgs A) {
 }
 
 // ---- fp32-row kernel (reference launchers): fragments straight from global -----------
+// A one-tile chunk is one memory latency per 16 rows plus the partial's
+// stores: every row's 2 KB loads are in flight together, from addresses that do
+// not wait for the mask (a row past the end or masked reads a valid row and is
+// zeroed). kDq workgroups share a chunk, each with its kD / kDq output dims and
+// the whole QK^T (a chunk's rows come from L2): four for few chunks, whose CUs
+// would idle, one for many, where the repeated QK^T would cost more. Over 128 +
+// 1025 rows: 28.7 us with loads branched on the mask and two-tile chunks, 23.1
+// with loads in flight and one-tile chunks, 20.0 with four workgroups a chunk.
 // kSepV: V rows come from f32_v_raw (the raw launcher with V != K); otherwise
 // the K fragments are also the V tile (MLA: K == V).
-template <bool kSepV>
+template <bool kSepV, int kDq>
 __global__ __launch_bounds__(256) void decode_f32_kernel(const DecodeArgs A) {
-    __shared__ half_t vt[kD * kVtStride];
+    constexpr int kDims = kD / kDq, kVb = kDims / 64;   // this workgroup's dims, as 64-dim blocks
+    __shared__ half_t vt[kDims * kVtStride];
     __shared__ long long s_start[kMaxProb + 1];
     stage_start(A, s_start);
 
@@ -1007,6 +1014,12 @@ __global__ __launch_bounds__(256) void decode_f32_kernel(const DecodeArgs A) {
     const int j = lane & 15;
     const int q = lane >> 4;
     const int head = wave * 16 + j;
+    const int vb0 = kDq > 1 ? kVb * (int)blockIdx.y : 0;
+    // the V^T blocks this wave writes: of both row halves (kDq 1: its two
+    // blocks), or of one half (kDq 4: one of the two blocks)
+    auto my_v = [&](int h2, int b) {
+        return kDq == 1 ? (b >> 1) == wave : b == vb0 + (wave & 1) && h2 == (wave >> 1);
+    };
 
     long long g0 = (long long)blockIdx.x * A.chunk;
     const long long g1 = min(g0 + (long long)A.chunk, A.total);
@@ -1023,39 +1036,51 @@ __global__ __launch_bounds__(256) void decode_f32_kernel(const DecodeArgs A) {
         const long long r1 = min(seg_end - s_start[p], A.count[p]);
 
         half8_t qh[16], ql[16];
-        load_q<true>(A, p, head, q, qh, ql);
-        SegState S;
+        load_q(A, p, head, q, qh, ql);
+        SegState<kDims / 16> S;
         seg_init(S);
 
         for (long long rb = r0; rb < r1; rb += kTile) {
             __syncthreads();   // previous tile's P.V reads of vt are done
+            // one copy of a row half's code: a chunk of one tile runs it twice, and
+            // instruction fetch is a good part of so short a kernel
             float4_t acc[2];
-#pragma unroll
+#pragma unroll 1
             for (int h2 = 0; h2 < 2; ++h2) {
-                acc[h2] = float4_t{0, 0, 0, 0};
+                float4_t sum = float4_t{0, 0, 0, 0};
                 const long long r = rb + 16 * h2 + j;
-                const bool valid = r < r1 && row_allowed(r);
-                const float *frow = r < A.f32_n_raw ? A.f32_raw + r * kD
-                                                    : A.f32_comp + (r - A.f32_n_raw) * kD;
+                const long long rc = min(r, r1 - 1);
+                const float *frow = rc < A.f32_n_raw ? A.f32_raw + rc * kD : A.f32_comp + (rc - A.f32_n_raw) * kD;
                 const int prow = vt_pos(16 * h2 + j);
+                float4_t kf[8][4], vf[kSepV ? 2 : 1][4];
+#pragma unroll
+                for (int b = 0; b < 8; ++b) load_f32_raw(frow, b, q, kf[b]);
+                if (kSepV)
+#pragma unroll
+                    for (int i = 0; i < (kDq == 1 ? 2 : 1); ++i)
+                        load_f32_raw(A.f32_v_raw + rc * kD, kDq == 1 ? 2 * wave + i : vb0 + (wave & 1), q, vf[i]);
+                const bool valid = r < r1 && row_allowed(rc);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int b = 0; b < 8; ++b) {
                     half8_t a0, a1;
-                    load_f32_block(frow, b, q, valid, a0, a1);
-                    acc[h2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, qh[2 * b], acc[h2], 0, 0, 0);
-                    acc[h2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, qh[2 * b + 1], acc[h2], 0, 0, 0);
-                    acc[h2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, ql[2 * b], acc[h2], 0, 0, 0);
-                    acc[h2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, ql[2 * b + 1], acc[h2], 0, 0, 0);
-                    if ((b >> 1) == wave) {
+                    round_f32_block(kf[b], valid, a0, a1);
+                    sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, qh[2 * b], sum, 0, 0, 0);
+                    sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, qh[2 * b + 1], sum, 0, 0, 0);
+                    sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, ql[2 * b], sum, 0, 0, 0);
+                    sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, ql[2 * b + 1], sum, 0, 0, 0);
+                    if (my_v(h2, b)) {
                         if (kSepV) {
                             half8_t v0, v1;
-                            load_f32_block(A.f32_v_raw + r * kD, b, q, valid, v0, v1);
-                            vt_write(vt, b, q, prow, v0, v1);
+                            round_f32_block(vf[kDq == 1 ? b & 1 : 0], valid, v0, v1);
+                            vt_write(vt, b - vb0, q, prow, v0, v1);
                         } else {
-                            vt_write(vt, b, q, prow, a0, a1);
+                            vt_write(vt, b - vb0, q, prow, a0, a1);
                         }
                     }
                 }
+                if (h2 == 0) acc[0] = sum;
+                else acc[1] = sum;
             }
             const half8_t pf = softmax_tile(acc, A.kq_log2, q, S, [&](int h2, int r) {
                 const long long row = rb + 16 * h2 + 4 * q + r;
@@ -1064,11 +1089,11 @@ __global__ __launch_bounds__(256) void decode_f32_kernel(const DecodeArgs A) {
             __syncthreads();   // V^T tile complete
             pv_tile(vt, pf, j, q, S);
         }
-        emit_partial(A, (long long)blockIdx.x * A.s_max + slot_s, wave, j, q, head, p, S);
+        emit_partial(A, (long long)blockIdx.x * A.s_max + slot_s, wave, j, q, head, p, 64 * vb0, S);
         ++slot_s;
         g0 = seg_end;
     }
-    if (threadIdx.x == 0)
+    if (threadIdx.x == 0 && vb0 == 0)
         for (int s2 = slot_s; s2 < A.s_max; ++s2) A.ws_prob[(long long)blockIdx.x * A.s_max + s2] = -1;
 }
 
@@ -2453,12 +2478,19 @@ __global__ __launch_bounds__(128) void decode_merge_kernel(const DecodeArgs A) {
         __syncthreads();
         const int nb = (int)std::min<long long>(128, n_slot - base);
         const float *o0 = A.ws_o + (s0 + base) * (kH * kD) + h * kD + 4 * tid;
-#pragma unroll 16
-        for (int j = 0; j < nb; ++j) {
-            const float c = s_sc[j];
-            const float4_t o = *reinterpret_cast<const float4_t *>(o0 + (long long)j * (kH * kD));
-            den += s_dl[j];
-            acc = c != 0.0f ? acc + o * c : acc;   // a select: unused slots may hold anything
+        // eight slots' loads in flight; slots past nb have scale 0
+#pragma unroll 1
+        for (int j = 0; j < nb; j += 8) {
+            float4_t o[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                o[i] = *reinterpret_cast<const float4_t *>(o0 + (long long)min(j + i, nb - 1) * (kH * kD));
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float c = s_sc[j + i];
+                den += s_dl[j + i];
+                acc = c != 0.0f ? acc + o[i] * c : acc;   // a select: unused slots may hold anything
+            }
         }
     }
     // a problem that met a row outside the cache gets NaN, never a plausible value
@@ -2548,11 +2580,18 @@ __global__ __launch_bounds__(kMergeThreads) void decode_merge_wide_kernel(const 
         __syncthreads();
         const int nb = (int)min((long long)kMergeThreads, n_slot - base);
         const float *ob = o_base + (s0 + base) * (kH * kD);
-#pragma unroll 8
-        for (int jj = wave; jj < nb; jj += 4) {
-            const float c = s_sc[jj];
-            const float4_t o = *reinterpret_cast<const float4_t *>(ob + (long long)jj * (kH * kD));
-            acc = c != 0.0f ? acc + o * c : acc;   // a select: unused slots may hold anything
+        // eight slots' loads in flight; slots past nb have scale 0
+#pragma unroll 1
+        for (int jj = wave; jj < nb; jj += 32) {
+            float4_t o[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                o[i] = *reinterpret_cast<const float4_t *>(ob + (long long)min(jj + 4 * i, nb - 1) * (kH * kD));
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float c = s_sc[jj + 4 * i];
+                acc = c != 0.0f ? acc + o[i] * c : acc;   // a select: unused slots may hold anything
+            }
         }
     }
     const float den = block_reduce(den_part, false) + __builtin_amdgcn_exp2f(sink - mx);
@@ -2731,10 +2770,15 @@ int launch(DecodeArgs &A, const Plan &pl, hipStream_t st, int phases = 3,
         }
         else if (kFp8)
             hipLaunchKernelGGL(decode_fp8_kernel<kQf32>, dim3(pl.n_wg), dim3(256), 0, st, A);
-        else if (A.f32_v_raw)
-            hipLaunchKernelGGL(decode_f32_kernel<true>, dim3(pl.n_wg), dim3(256), 0, st, A);
+        else if (pl.n_wg * 4 <= 2 * num_cus()) {   // few chunks: four workgroups each
+            if (A.f32_v_raw)
+                hipLaunchKernelGGL((decode_f32_kernel<true, 4>), dim3(pl.n_wg, 4), dim3(256), 0, st, A);
+            else
+                hipLaunchKernelGGL((decode_f32_kernel<false, 4>), dim3(pl.n_wg, 4), dim3(256), 0, st, A);
+        } else if (A.f32_v_raw)
+            hipLaunchKernelGGL((decode_f32_kernel<true, 1>), dim3(pl.n_wg), dim3(256), 0, st, A);
         else
-            hipLaunchKernelGGL(decode_f32_kernel<false>, dim3(pl.n_wg), dim3(256), 0, st, A);
+            hipLaunchKernelGGL((decode_f32_kernel<false, 1>), dim3(pl.n_wg), dim3(256), 0, st, A);
         const int e = hip_status(hipGetLastError());
         if (e) return e;
     }
@@ -2891,14 +2935,19 @@ extern "C" long long ds4hip_flash_attn_q_prep_words(void) { return kQPrepWords; 
 // partials live in a workspace: the caller's (the _prealloc forms), or the
 // library's per-stream scratch (see stream_scratch).
 namespace {
-Plan f32_plan(long long n_rows) { return make_plan(&n_rows, 1, 2, 0, false); }
+// One-tile chunks; a caller's workspace that holds only the two-tile plan's
+// partials (one sized for another row count) gets that plan.
+Plan f32_plan(long long n_rows, int min_chunk = kMinChunkF32) {
+    return make_plan(&n_rows, 1, 2, 0, false, min_chunk);
+}
 
 int run_f32(const float *Q, const float *raw, const float *v_raw, int n_raw, const float *comp,
             int n_comp, const int32_t *allowed, const float *sinks, float *out, void *ws,
             size_t ws_bytes, hipStream_t st, const Plan *plan = nullptr) {
     DecodeArgs A = {};
     A.count[0] = (long long)n_raw + n_comp;
-    const Plan pl = plan ? *plan : f32_plan(A.count[0]);
+    Plan pl = plan ? *plan : f32_plan(A.count[0]);
+    if (!plan && ws && ws_bytes < pl.ws_bytes) pl = f32_plan(A.count[0], kMinChunk);
     A.start[0] = pl.start[0];
     A.start[1] = pl.start[1];
     if (!ws) {
@@ -3037,7 +3086,7 @@ extern "C" int ds4hip_flash_attn_decode_mixed_f32_noalloc(
         (long long)n_raw + n_comp > kNoAllocMaxRows)
         return ds4hip_set_last_error(kEINVAL);
     const long long n = (long long)n_raw + n_comp;
-    const Plan pl = make_plan(&n, 1, 2, kNoAllocSlots, false);
+    const Plan pl = make_plan(&n, 1, 2, kNoAllocSlots, false, kMinChunkF32);
     if (pl.ws_bytes > kNoAllocScratchBytes) return ds4hip_set_last_error(kEINVAL);
     void *ws = nullptr;
     const int rc = scratch_ptr(&ws);
