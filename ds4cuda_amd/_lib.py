@@ -101,6 +101,7 @@ SIGNATURES: dict[str, list] = {
     "ds4hip_session_chunk_step_workspace_bytes": [_vp, _i, _i],
     "ds4hip_session_chunk_step": [_vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp],
     "ds4hip_session_push_raw_rows": [_vp, _i, _vp, _i, _vp],
+    "ds4hip_session_emit_f32": [_vp, _i, _i, _vp, _vp, _vp, _vp],
     "ds4hip_session_save_to_disk": [_vp, _vp, _i, C.c_char_p],
     "ds4hip_session_load_from_disk": [_vp, C.c_char_p, C.POINTER(_i), C.POINTER(_i)],
     "ds4hip_ds4cudak_probe": [C.c_char_p, _vp],

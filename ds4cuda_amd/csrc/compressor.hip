@@ -16,6 +16,7 @@
 #include "ds4hip_common.h"
 #include "step_bodies.h"
 #include "../../include/ds4hip.h"
+#include "../../include/ds4hip_session.h"
 
 #include <cmath>
 
@@ -76,6 +77,31 @@ __global__ __launch_bounds__(512) void comp_emit_kernel(float *__restrict__ stat
                                                         float *__restrict__ emit_out, int head_dim,
                                                         int ratio, int is_attn, RopeArgs R) {
     emit_body(state_kv, state_score, w_norm, emit_out, head_dim, ratio, is_attn, R);
+}
+
+// A token's emits of one layer with their pushes: workgroup 0 the attention
+// compressor's row, which its first wave then quantizes into the cache row,
+// workgroup 1 (indexer layers) the indexer key, straight into its key row.
+// Four launches of about 5 us each, one after the other, before.
+struct TokenEmitArgs {
+    float *state_kv[2], *state_score[2], *emit[2];
+    const float *w_norm[2];
+    uint8_t *codes;
+    int8_t *sexp;
+    uint16_t *tail;
+    long long row;
+    int ratio;
+    RopeArgs rope;
+};
+__global__ __launch_bounds__(512) void token_emit_kernel(const TokenEmitArgs A) {
+    const int job = blockIdx.x;
+    const int head_dim = job ? DS4HIP_INDEXER_HEAD_DIM : DS4HIP_HEAD_DIM;
+    emit_body(A.state_kv[job], A.state_score[job], A.w_norm[job], A.emit[job], head_dim, A.ratio, job == 0 ? 1 : 0,
+              A.rope);
+    // emit_body's last barrier orders the row's stores before these loads
+    if (job == 0 && threadIdx.x < 64)
+        fp8_row_body<false>(A.emit[0], nullptr, A.codes, A.sexp, A.tail, 0, DS4HIP_HEAD_DIM, DS4HIP_N_ROT, A.row,
+                            threadIdx.x);
 }
 
 // ---- batched step: n_seq sequences, one position each ----------------------------------
@@ -203,6 +229,40 @@ extern "C" int ds4hip_compressor_emit_f32(int is_attn, const float *w_norm_f32, 
                        w_norm_f32, emit_out, head_dim_out, compress_ratio, is_attn ? 1 : 0,
                        rope_args(il, pos + 1 - compress_ratio));
     return ds4hip_set_last_error(hip_status(hipGetLastError()));
+}
+
+extern "C" int ds4hip_session_emit_f32(ds4hip_session_state *s, int il, int pos, const float *w_comp_norm,
+                                       const float *w_idx_norm, float *emit_scratch, void *stream) {
+    if (!s || !s->arena_base || il < 0 || il >= DS4HIP_N_LAYER || pos < 0 || !w_comp_norm || !emit_scratch)
+        return ds4hip_set_last_error(kEINVAL);
+    ds4hip_layer_state *L = &s->layers[il];
+    if (!L->compress_ratio || (pos + 1) % L->compress_ratio || (L->has_indexer && !w_idx_norm))
+        return ds4hip_set_last_error(kEINVAL);
+    if (L->n_comp >= L->cap_comp || (L->has_indexer && L->n_index_comp >= L->cap_comp))
+        return ds4hip_set_last_error(DS4HIP_ENOSPC);
+    TokenEmitArgs A{};
+    A.state_kv[0] = L->attn_state_kv;
+    A.state_score[0] = L->attn_state_score;
+    A.emit[0] = emit_scratch;
+    A.w_norm[0] = w_comp_norm;
+    A.codes = s->codes;
+    A.sexp = s->sexp;
+    A.tail = s->tail;
+    A.row = L->row_base + L->n_comp;
+    A.ratio = L->compress_ratio;
+    A.rope = rope_args(il, pos + 1 - L->compress_ratio);
+    if (L->has_indexer) {
+        A.state_kv[1] = L->index_state_kv;
+        A.state_score[1] = L->index_state_score;
+        A.emit[1] = L->index_comp_kv + (size_t)L->n_index_comp * DS4HIP_INDEXER_HEAD_DIM;
+        A.w_norm[1] = w_idx_norm;
+    }
+    hipLaunchKernelGGL(token_emit_kernel, dim3(L->has_indexer ? 2 : 1), dim3(512), 0, (hipStream_t)stream, A);
+    const int rc = hip_status(hipGetLastError());
+    if (rc) return ds4hip_set_last_error(rc);
+    ++L->n_comp;
+    if (L->has_indexer) ++L->n_index_comp;
+    return 0;
 }
 
 extern "C" int ds4hip_compressor_decode_step_f32_prealloc(

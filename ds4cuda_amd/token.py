@@ -307,14 +307,9 @@ class TokenSlice:
         # the decode query, converted for Step 13's kernel
         P.qp_q, P.qp_out = _ptr(q_cur[il]), _ptr(self.q_pre)
         call("ds4hip_token_prologue_f32", C.byref(P), st)
-        if emit:   # the emits and their row pushes
-            call("ds4hip_compressor_emit_f32", 1, _ptr(w["comp_norm"]), HEAD_DIM, r, pos, il,
-                 _vp(L.attn_state_kv), _vp(L.attn_state_score), _ptr(self.emit), st)
-            sess.push_comp(il, self.emit, stream=stream)
-            if r == 4:
-                call("ds4hip_compressor_emit_f32", 0, _ptr(w["idx_norm"]), IDX_DIM, r, pos, il,
-                     _vp(L.index_state_kv), _vp(L.index_state_score), _ptr(self.emit_i), st)
-                sess.push_index_comp(il, self.emit_i, stream=stream)
+        if emit:   # the emits and their row pushes, one launch
+            call("ds4hip_session_emit_f32", C.byref(s), il, pos, _ptr(w["comp_norm"]), _ptr(w.get("idx_norm")),
+                 _ptr(self.emit), st)
         n_sel = -1
         L = s.layers[il]
         if select:

@@ -208,6 +208,16 @@ int ds4hip_session_chunk_step(ds4hip_session_state *s, int il, int p0, int n_tok
                               int *n_comp_tok, int *n_sel_tok, void *workspace, size_t workspace_bytes,
                               void *stream);
 
+/* A token's emits of layer il at pos, (pos + 1) % ratio == 0, after its
+ * projections are in the state rows: ds4hip_compressor_emit_f32 of the
+ * attention compressor (and on indexer layers of the indexer compressor) and
+ * ds4hip_session_push_comp / _push_index_comp of their rows, bit for bit, in one
+ * launch (no counterpart in the reference). emit_scratch [512] receives the
+ * attention compressor's row; w_idx_norm is read on indexer layers only. -28
+ * when a row does not fit (nothing is changed). */
+int ds4hip_session_emit_f32(ds4hip_session_state *s, int il, int pos, const float *w_comp_norm,
+                            const float *w_idx_norm, float *emit_scratch, void *stream);
+
 /* ds4hip_session_push_raw for n_rows <= cap_raw rows [n_rows][512], in order. */
 int ds4hip_session_push_raw_rows(ds4hip_session_state *s, int il, const float *kv, int n_rows, void *stream);
 
