@@ -1735,7 +1735,15 @@ __device__ inline float xmax_16_32_raw(float v) {
 // kGather: 0 direct rows; 1 physical rows from the phys array (phys_kernel
 // ran: pages and / or row lists); 2 the int32 row list itself (no pages: row
 // = the problem's base + entry, clamped into the cache)
-template <bool kPLo, bool kLean, int kQf32 = 0, int kGather = 0>
+// kShort: no segment is longer than kFsLead tiles (chunks of at most that): the
+// prologue's copies are all there are, so the tile loop issues and waits for
+// none. The ring of the other form always copies kFsLead tiles ahead, past the
+// segment's end too (its last row again), which keeps its waits at one count;
+// a copy costs its issue in the address unit, 0.5 us a tile, and a one-tile
+// segment that copied six took a token's gathered decodes 12.0 us, 10.2 now.
+// (The condition inside the one loop instead cost a 4096-row decode 62.6 ->
+// 63.0 us and 16 paged problems 54.3 -> 56.6; per tile, 66.1.)
+template <bool kPLo, bool kLean, int kQf32 = 0, int kGather = 0, bool kShort = false>
 __global__ __launch_bounds__(512, 1) void decode_flat_kernel(const DecodeArgs A) {
     static_assert(kLean || !kQf32, "fp32 Q takes the lean form");
     // Q parts on the scaled FP8 MFMA: a bf16 Q (8 significant bits) fits in
@@ -2078,7 +2086,7 @@ __global__ __launch_bounds__(512, 1) void decode_flat_kernel(const DecodeArgs A)
                         __builtin_amdgcn_global_load_lds(reinterpret_cast<const uint8_t *>(A.tail) + rr[k] * (2 * kRot) + c_off[k],
                                                          st + 1024 * n, 16, 0, 0);
                 }
-                if (c == 0) {
+                if (!kShort && c == 0) {   // kShort: no later tile
                     int ln2 = lane;
                     asm volatile("" : "+v"(ln2));
                     if constexpr (kGather == 1) {
@@ -2319,7 +2327,8 @@ __global__ __launch_bounds__(512, 1) void decode_flat_kernel(const DecodeArgs A)
                 else
                     asm volatile("s_waitcnt vmcnt(%0)" :: "n"(5 * (kFsLead - 1)) : "memory");
             };
-            // prologue: tiles 0 .. kFsLead - 1; tile 0 lands before the first barrier
+            // prologue: tiles 0 .. kFsLead - 1 (kShort: those there are, all landed before
+            // the first barrier); tile 0 lands before the first barrier
             if constexpr (kGather != 0) {
                 // their rows straight from the phys array (or the row list), all
                 // loaded before any copy
@@ -2328,6 +2337,7 @@ __global__ __launch_bounds__(512, 1) void decode_flat_kernel(const DecodeArgs A)
                 for (int u = 0; u < kFsLead; ++u)
 #pragma unroll
                     for (int k = 0; k < 5; ++k) {
+                        if (kShort && u >= n_tiles) continue;
                         const int e = min(kTile * u + c_row[k], seg_last);
                         if constexpr (kGather == 1) {
                             const long long v = A.phys[g0 + e];
@@ -2340,21 +2350,26 @@ __global__ __launch_bounds__(512, 1) void decode_flat_kernel(const DecodeArgs A)
                         }
                     }
 #pragma unroll
-                for (int u = 0; u < kFsLead; ++u) issue_rows(u, rr[u]);
+                for (int u = 0; u < kFsLead; ++u)
+                    if (!kShort || u < n_tiles) issue_rows(u, rr[u]);
                 report_bad();
             } else {
 #pragma unroll
-                for (int u = 0; u < kFsLead; ++u) issue(u);
+                for (int u = 0; u < kFsLead; ++u)
+                    if (!kShort || u < n_tiles) issue(u);
             }
-            wait_ring();
+            if constexpr (kShort) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            else wait_ring();
             lds_barrier();
             // interval u: copies of u + kFsLead, P . V(u - 2); before the barrier
             // that ends it, tile u + 1 has landed (this wave's copies)
             for (int u = 0; u < n_tiles + 2; ++u) {
-                issue(u + kFsLead);
-                report_bad();
+                if constexpr (!kShort) {
+                    issue(u + kFsLead);
+                    report_bad();
+                }
                 if (u >= 2) pv(u - 2);
-                wait_ring();
+                if constexpr (!kShort) wait_ring();
                 lds_barrier();
             }
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -2703,6 +2718,16 @@ void carve(DecodeArgs &A, void *ws, const Plan &pl) {
     A.phys = reinterpret_cast<long long *>(c);   // used only by gathered steps (reset below)
 }
 
+// The flat-stage kernel: the form without a copy ring when no chunk is longer
+// than the copies' lead.
+template <bool kPLo, int kQf32, int kGather>
+void launch_flat(const DecodeArgs &A, const Plan &pl, hipStream_t st) {
+    if (pl.chunk <= kFsLead * kTile)
+        hipLaunchKernelGGL((decode_flat_kernel<kPLo, true, kQf32, kGather, true>), dim3(pl.n_wg), dim3(512), 0, st, A);
+    else
+        hipLaunchKernelGGL((decode_flat_kernel<kPLo, true, kQf32, kGather>), dim3(pl.n_wg), dim3(512), 0, st, A);
+}
+
 // Kernel for the bf16-Q partials, chosen per call (ds4hip_decode_opts): direct
 // rows with one f16 P run the flat-stage kernel (its lean form) unless the
 // caller asks for the register-load kernel; row lists, pages and the
@@ -2712,13 +2737,13 @@ template <int kMode>
 void launch_ws(const DecodeArgs &A, const Plan &pl, hipStream_t st, const ds4hip_decode_opts &o) {
     if (kMode < 2 && o.kernel != DS4HIP_DECODE_KERNEL_REGLOAD) {
         if (kMode == 0 && o.exact_p)
-            hipLaunchKernelGGL((decode_flat_kernel<true, true>), dim3(pl.n_wg), dim3(512), 0, st, A);
+            launch_flat<true, 0, 0>(A, pl, st);
         else if (kMode == 0)
-            hipLaunchKernelGGL((decode_flat_kernel<false, true>), dim3(pl.n_wg), dim3(512), 0, st, A);
+            launch_flat<false, 0, 0>(A, pl, st);
         else if (o.exact_p)
-            hipLaunchKernelGGL((decode_flat_kernel<true, true, false, 1>), dim3(pl.n_wg), dim3(512), 0, st, A);
+            launch_flat<true, 0, 1>(A, pl, st);
         else
-            hipLaunchKernelGGL((decode_flat_kernel<false, true, false, 1>), dim3(pl.n_wg), dim3(512), 0, st, A);
+            launch_flat<false, 0, 1>(A, pl, st);
         return;
     }
     if (o.exact_p)
@@ -2756,17 +2781,17 @@ int launch(DecodeArgs &A, const Plan &pl, hipStream_t st, int phases = 3,
             // fp32 Q: the flat-stage kernel with Q in three FP8 parts and, as
             // every fp32-Q decode, P as f16 hi + lo
             if (q_pre && idx_only)
-                hipLaunchKernelGGL((decode_flat_kernel<true, true, 2, 2>), dim3(pl.n_wg), dim3(512), 0, st, A);
+                launch_flat<true, 2, 2>(A, pl, st);
             else if (q_pre && A.phys)
-                hipLaunchKernelGGL((decode_flat_kernel<true, true, 2, 1>), dim3(pl.n_wg), dim3(512), 0, st, A);
+                launch_flat<true, 2, 1>(A, pl, st);
             else if (q_pre)
-                hipLaunchKernelGGL((decode_flat_kernel<true, true, 2, 0>), dim3(pl.n_wg), dim3(512), 0, st, A);
+                launch_flat<true, 2, 0>(A, pl, st);
             else if (idx_only)
-                hipLaunchKernelGGL((decode_flat_kernel<true, true, 1, 2>), dim3(pl.n_wg), dim3(512), 0, st, A);
+                launch_flat<true, 1, 2>(A, pl, st);
             else if (A.phys)
-                hipLaunchKernelGGL((decode_flat_kernel<true, true, 1, 1>), dim3(pl.n_wg), dim3(512), 0, st, A);
+                launch_flat<true, 1, 1>(A, pl, st);
             else
-                hipLaunchKernelGGL((decode_flat_kernel<true, true, 1, 0>), dim3(pl.n_wg), dim3(512), 0, st, A);
+                launch_flat<true, 1, 0>(A, pl, st);
         }
         else if (kFp8)
             hipLaunchKernelGGL(decode_fp8_kernel<kQf32>, dim3(pl.n_wg), dim3(256), 0, st, A);
