@@ -2432,6 +2432,12 @@ __global__ __launch_bounds__(256) void phys_kernel(const DecodeArgs A) {
 // L2 round trip per slot); the slots' scale factors then go through LDS and
 // thread t accumulates dims 4t..4t+3 over the slots in slot order, several
 // slots' 16-byte loads in flight at once.
+//
+// kMany: many workgroups per CU hide each other's loads, so the slots are read
+// one by one without the repeated rows of a short group of eight (43 problems of
+// six chunks 12.0 us, 14.6 in groups); one problem's 64 workgroups are bound by
+// their own chain and code (8.4 us slot by slot, unrolled; 6.9 in groups).
+template <bool kMany>
 __global__ __launch_bounds__(128) void decode_merge_kernel(const DecodeArgs A) {
     __shared__ float s_sc[128], s_dl[128];
     __shared__ float s_mx[2];
@@ -2493,6 +2499,16 @@ __global__ __launch_bounds__(128) void decode_merge_kernel(const DecodeArgs A) {
         __syncthreads();
         const int nb = (int)std::min<long long>(128, n_slot - base);
         const float *o0 = A.ws_o + (s0 + base) * (kH * kD) + h * kD + 4 * tid;
+        if constexpr (kMany) {
+#pragma unroll 16
+            for (int j = 0; j < nb; ++j) {
+                const float c = s_sc[j];
+                const float4_t o = *reinterpret_cast<const float4_t *>(o0 + (long long)j * (kH * kD));
+                den += s_dl[j];
+                acc = c != 0.0f ? acc + o * c : acc;   // as below
+            }
+            continue;
+        }
         // eight slots' loads in flight; slots past nb have scale 0
 #pragma unroll 1
         for (int j = 0; j < nb; j += 8) {
@@ -2521,6 +2537,7 @@ __global__ __launch_bounds__(128) void decode_merge_kernel(const DecodeArgs A) {
 // slots (slot j to wave j mod 4, in slot order), thread t dims 4t..4t+3 of the
 // half, several slots' 16-byte loads in flight, and the four waves' sums are
 // added in wave order: a fixed order, so the result is deterministic.
+constexpr int kMergeManyProblems = 8;   // 64 merges each: two workgroups per CU
 constexpr int kMergeThreads = 256;
 constexpr long long kMergeWideSlots = 8;   // chunks per problem above which the wide merge runs
 __global__ __launch_bounds__(kMergeThreads) void decode_merge_wide_kernel(const DecodeArgs A) {
@@ -2597,11 +2614,11 @@ __global__ __launch_bounds__(kMergeThreads) void decode_merge_wide_kernel(const 
         const float *ob = o_base + (s0 + base) * (kH * kD);
         // eight slots' loads in flight; slots past nb have scale 0
 #pragma unroll 1
-        for (int jj = wave; jj < nb; jj += 32) {
+        for (int jj = __builtin_amdgcn_readfirstlane(wave); jj < nb; jj += 32) {
             float4_t o[8];
 #pragma unroll
             for (int i = 0; i < 8; ++i)
-                o[i] = *reinterpret_cast<const float4_t *>(ob + (long long)min(jj + 4 * i, nb - 1) * (kH * kD));
+                o[i] = jj + 4 * i < nb ? *reinterpret_cast<const float4_t *>(ob + (long long)(jj + 4 * i) * (kH * kD)) : float4_t{0, 0, 0, 0};
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const float c = s_sc[jj + 4 * i];
@@ -2821,8 +2838,10 @@ int launch(DecodeArgs &A, const Plan &pl, hipStream_t st, int phases = 3,
         }
         if (max_slots > kMergeWideSlots)
             hipLaunchKernelGGL(decode_merge_wide_kernel, dim3(A.n_prob, kH, 2), dim3(kMergeThreads), 0, st, A);
+        else if (A.n_prob >= kMergeManyProblems)
+            hipLaunchKernelGGL(decode_merge_kernel<true>, dim3(A.n_prob, kH), dim3(128), 0, st, A);
         else
-            hipLaunchKernelGGL(decode_merge_kernel, dim3(A.n_prob, kH), dim3(128), 0, st, A);
+            hipLaunchKernelGGL(decode_merge_kernel<false>, dim3(A.n_prob, kH), dim3(128), 0, st, A);
     }
     return hip_status(hipGetLastError());
 }
