@@ -52,9 +52,8 @@ constexpr int kNope = kD - kRot; // 448 FP8-coded dims, 7 scale blocks
 constexpr int kTile = 32;        // rows per tile
 constexpr int kVtStride = 40;    // halves per V^T line (32 rows + 8 pad)
 constexpr int kMaxProb = 128;
-constexpr int kMinChunk = 2 * kTile;       // the register-load kernels run tiles in pairs
+constexpr int kMinChunk = 2 * kTile;       // the register-load kernels run tiles in pairs; the fp32-row kernel (below)
 constexpr int kMinChunkFlat = kTile;       // the flat-stage kernel: one tile is a whole chunk
-constexpr int kMinChunkF32 = kTile;        // and the fp32-row kernel
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLazyLog2 = 8.0f;   // decode softmax: reference point slack (log2 units)
 constexpr int kFp8WgPerCu = 1;   // the FP8 kernel's LDS ring allows one workgroup per CU
@@ -992,14 +991,16 @@ __global__ __launch_bounds__(256) void decode_fp8_kernel(const DecodeArgs A) {
 }
 
 // ---- fp32-row kernel (reference launchers): fragments straight from global -----------
-// A one-tile chunk is one memory latency per 16 rows plus the partial's
-// stores: every row's 2 KB loads are in flight together, from addresses that do
-// not wait for the mask (a row past the end or masked reads a valid row and is
+// A short chunk is one memory latency per 16 rows plus the partial's stores:
+// every row's 2 KB loads are in flight together, from addresses that do not
+// wait for the mask (a row past the end or masked reads a valid row and is
 // zeroed). kDq workgroups share a chunk, each with its kD / kDq output dims and
 // the whole QK^T (a chunk's rows come from L2): four for few chunks, whose CUs
-// would idle, one for many, where the repeated QK^T would cost more. Over 128 +
-// 1025 rows: 28.7 us with loads branched on the mask and two-tile chunks, 23.1
-// with loads in flight and one-tile chunks, 20.0 with four workgroups a chunk.
+// would idle, one for many, where the repeated QK^T would cost more.
+// P enters P . V as one f16 relative to the chunk's running maximum, so where
+// the chunks are cut is part of the result: shorter ones move the rounding of
+// the heaviest weights (1e-5 of the output on rows with outliers). They stay at
+// two tiles, also where one would be faster.
 // kSepV: V rows come from f32_v_raw (the raw launcher with V != K); otherwise
 // the K fragments are also the V tile (MLA: K == V).
 template <bool kSepV, int kDq>
@@ -2824,7 +2825,10 @@ int launch(DecodeArgs &A, const Plan &pl, hipStream_t st, int phases = 3,
         }
         else if (kFp8)
             hipLaunchKernelGGL(decode_fp8_kernel<kQf32>, dim3(pl.n_wg), dim3(256), 0, st, A);
-        else if (pl.n_wg * 4 <= 2 * num_cus()) {   // few chunks: four workgroups each
+        else if (pl.n_wg * 4 <= num_cus()) {
+            // few chunks: four workgroups each, as long as every one has a CU of its
+            // own (its registers fill one). On both sides of the line, one against
+            // four: 4096 rows 40.4 -> 36.1 us, 4224 rows 40.5 -> 58.
             if (A.f32_v_raw)
                 hipLaunchKernelGGL((decode_f32_kernel<true, 4>), dim3(pl.n_wg, 4), dim3(256), 0, st, A);
             else
@@ -2993,19 +2997,14 @@ extern "C" long long ds4hip_flash_attn_q_prep_words(void) { return kQPrepWords; 
 // partials live in a workspace: the caller's (the _prealloc forms), or the
 // library's per-stream scratch (see stream_scratch).
 namespace {
-// One-tile chunks; a caller's workspace that holds only the two-tile plan's
-// partials (one sized for another row count) gets that plan.
-Plan f32_plan(long long n_rows, int min_chunk = kMinChunkF32) {
-    return make_plan(&n_rows, 1, 2, 0, false, min_chunk);
-}
+Plan f32_plan(long long n_rows) { return make_plan(&n_rows, 1, 2, 0, false); }
 
 int run_f32(const float *Q, const float *raw, const float *v_raw, int n_raw, const float *comp,
             int n_comp, const int32_t *allowed, const float *sinks, float *out, void *ws,
             size_t ws_bytes, hipStream_t st, const Plan *plan = nullptr) {
     DecodeArgs A = {};
     A.count[0] = (long long)n_raw + n_comp;
-    Plan pl = plan ? *plan : f32_plan(A.count[0]);
-    if (!plan && ws && ws_bytes < pl.ws_bytes) pl = f32_plan(A.count[0], kMinChunk);
+    const Plan pl = plan ? *plan : f32_plan(A.count[0]);
     A.start[0] = pl.start[0];
     A.start[1] = pl.start[1];
     if (!ws) {
@@ -3144,7 +3143,7 @@ extern "C" int ds4hip_flash_attn_decode_mixed_f32_noalloc(
         (long long)n_raw + n_comp > kNoAllocMaxRows)
         return ds4hip_set_last_error(kEINVAL);
     const long long n = (long long)n_raw + n_comp;
-    const Plan pl = make_plan(&n, 1, 2, kNoAllocSlots, false, kMinChunkF32);
+    const Plan pl = make_plan(&n, 1, 2, kNoAllocSlots, false);
     if (pl.ws_bytes > kNoAllocScratchBytes) return ds4hip_set_last_error(kEINVAL);
     void *ws = nullptr;
     const int rc = scratch_ptr(&ws);

@@ -78,3 +78,46 @@ def test_workspace_sized_for_another_row_count(gpu):
         torch.cuda.synchronize()
         if rc == 0:
             check(out.cpu().numpy(), reference(q, k, k, sinks.astype(np.float64)))
+
+
+def chunked_f16_p(q, k, sinks, rows):
+    """The decode's rounding in fp64: chunks of `rows` rows in tiles of 32, P as
+    one f16 relative to the chunk's maximum so far, l of the unrounded P."""
+    k = k.astype(np.float16).astype(np.float64)
+    s = q.astype(np.float64) @ k.T / np.sqrt(512.0) * np.log2(np.e)
+    parts = []
+    for c in range(0, len(k), rows):
+        m, l, o = np.full(64, -np.inf), np.zeros(64), np.zeros((64, 512))
+        for t in range(c, min(c + rows, len(k)), 32):
+            st = s[:, t:min(t + 32, c + rows)]
+            m_new = np.maximum(m, st.max(1))
+            p, a = np.exp2(st - m_new[:, None]), np.exp2(m - m_new)
+            o = o * a[:, None] + p.astype(np.float16).astype(np.float64) @ k[t:t + st.shape[1]]
+            l, m = l * a + p.sum(1), m_new
+        parts.append((m, l, o))
+    top = np.maximum(np.max([m for m, _, _ in parts], 0), sinks * np.log2(np.e))
+    w = [np.exp2(m - top) for m, _, _ in parts]
+    den = sum(x * l for x, (_, l, _) in zip(w, parts)) + np.exp2(sinks * np.log2(np.e) - top)
+    return sum(x[:, None] * o for x, (_, _, o) in zip(w, parts)) / den[:, None]
+
+
+@pytest.mark.parametrize("n", [200, 1153, 4000, 8192])
+def test_rounding_of_two_tile_chunks(gpu, n):
+    """Where the chunks are cut is part of the result: the outputs are those of
+    two-tile chunks, not of one-tile ones."""
+    q, k, _, sinks = inputs(n, 60 + n)
+    q = 2.0 * q
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)
+    kt = t(k)
+    out = torch.full((64, 512), float("nan"), device=gpu)
+    ops.launch_flash_attn_decode_raw_f32(t(q), kt, kt, t(sinks), out, 64, n, 512)
+    torch.cuda.synchronize()
+    s64 = sinks.astype(np.float64)
+    two, one = chunked_f16_p(q, k, s64, 64), chunked_f16_p(q, k, s64, 32)
+    rel = lambda a, b: np.linalg.norm(a - b, axis=1) / np.linalg.norm(b, axis=1)
+    # fp32 sums of 512 products move a score by about 1e-6, and with it an output
+    # by less than 3e-6, except where a weight crosses an f16 midpoint (2^-11 of
+    # that weight): so most heads, not all. The other cut moves half of them or more.
+    got = out.cpu().numpy()
+    assert np.median(rel(one, two)) > 2e-5
+    assert np.percentile(rel(got, two), 40) <= 3e-6
