@@ -992,15 +992,18 @@ __global__ __launch_bounds__(256) void decode_fp8_kernel(const DecodeArgs A) {
 
 // ---- fp32-row kernel (reference launchers): fragments straight from global -----------
 // A short chunk is one memory latency per 16 rows plus the partial's stores:
-// every row's 2 KB loads are in flight together, from addresses that do not
-// wait for the mask (a row past the end or masked reads a valid row and is
-// zeroed). kDq workgroups share a chunk, each with its kD / kDq output dims and
+// every row's 2 KB loads are in flight together, and the mask that decides
+// which rows are read (a masked row's are skipped) is fetched a tile ahead.
+// kDq workgroups share a chunk, each with its kD / kDq output dims and
 // the whole QK^T (a chunk's rows come from L2): four for few chunks, whose CUs
 // would idle, one for many, where the repeated QK^T would cost more.
 // P enters P . V as one f16 relative to the chunk's running maximum, so where
 // the chunks are cut is part of the result: shorter ones move the rounding of
 // the heaviest weights (1e-5 of the output on rows with outliers). They stay at
 // two tiles, also where one would be faster.
+// Measured against loads that wait for the mask block by block: 128 rows 31.3
+// -> 27.6 us, 128 + 1025 rows with 512 allowed 32.6 -> 28.5 (31.9 with the
+// masked rows read), 128 + 16384 with 490 allowed 65.5 -> 54.0 (72.7).
 // kSepV: V rows come from f32_v_raw (the raw launcher with V != K); otherwise
 // the K fragments are also the V tile (MLA: K == V).
 template <bool kSepV, int kDq>
@@ -1036,12 +1039,20 @@ __global__ __launch_bounds__(256) void decode_f32_kernel(const DecodeArgs A) {
         const long long r0 = g0 - s_start[p];
         const long long r1 = min(seg_end - s_start[p], A.count[p]);
 
+        // whether the lane's row of a tile's row half takes part
+        auto takes_part = [&](long long r) {
+            int ok = r < r1;
+            if (!kSepV && ok && A.f32_allowed && r >= A.f32_n_raw) ok = A.f32_allowed[r - A.f32_n_raw];
+            return ok;
+        };
+        int ok0 = takes_part(r0 + j), ok1 = takes_part(r0 + 16 + j);
         half8_t qh[16], ql[16];
         load_q(A, p, head, q, qh, ql);
         SegState<kDims / 16> S;
         seg_init(S);
 
         for (long long rb = r0; rb < r1; rb += kTile) {
+            const int next0 = takes_part(rb + kTile + j), next1 = takes_part(rb + kTile + 16 + j);
             __syncthreads();   // previous tile's P.V reads of vt are done
             // one copy of a row half's code: a chunk of one tile runs it twice, and
             // instruction fetch is a good part of so short a kernel
@@ -1049,23 +1060,25 @@ __global__ __launch_bounds__(256) void decode_f32_kernel(const DecodeArgs A) {
 #pragma unroll 1
             for (int h2 = 0; h2 < 2; ++h2) {
                 float4_t sum = float4_t{0, 0, 0, 0};
-                const long long r = rb + 16 * h2 + j;
-                const long long rc = min(r, r1 - 1);
-                const float *frow = rc < A.f32_n_raw ? A.f32_raw + rc * kD : A.f32_comp + (rc - A.f32_n_raw) * kD;
+                // kSepV: rows have no mask; one past the end reads the last row
+                const long long r = kSepV ? min(rb + 16 * h2 + j, r1 - 1) : rb + 16 * h2 + j;
+                const bool ok = h2 ? ok1 : ok0;
+                const float *frow = r < A.f32_n_raw ? A.f32_raw + r * kD : A.f32_comp + (r - A.f32_n_raw) * kD;
                 const int prow = vt_pos(16 * h2 + j);
-                float4_t kf[8][4], vf[kSepV ? 2 : 1][4];
+                float4_t kf[8][4] = {}, vf[kSepV ? 2 : 1][4] = {};
+                if (kSepV || ok) {
 #pragma unroll
-                for (int b = 0; b < 8; ++b) load_f32_raw(frow, b, q, kf[b]);
-                if (kSepV)
+                    for (int b = 0; b < 8; ++b) load_f32_raw(frow, b, q, kf[b]);
+                    if (kSepV)
 #pragma unroll
-                    for (int i = 0; i < (kDq == 1 ? 2 : 1); ++i)
-                        load_f32_raw(A.f32_v_raw + rc * kD, kDq == 1 ? 2 * wave + i : vb0 + (wave & 1), q, vf[i]);
-                const bool valid = r < r1 && row_allowed(rc);
+                        for (int i = 0; i < (kDq == 1 ? 2 : 1); ++i)
+                            load_f32_raw(A.f32_v_raw + r * kD, kDq == 1 ? 2 * wave + i : vb0 + (wave & 1), q, vf[i]);
+                }
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int b = 0; b < 8; ++b) {
                     half8_t a0, a1;
-                    round_f32_block(kf[b], valid, a0, a1);
+                    round_f32_block(kf[b], !kSepV || ok, a0, a1);
                     sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, qh[2 * b], sum, 0, 0, 0);
                     sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, qh[2 * b + 1], sum, 0, 0, 0);
                     sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, ql[2 * b], sum, 0, 0, 0);
@@ -1073,7 +1086,7 @@ __global__ __launch_bounds__(256) void decode_f32_kernel(const DecodeArgs A) {
                     if (my_v(h2, b)) {
                         if (kSepV) {
                             half8_t v0, v1;
-                            round_f32_block(vf[kDq == 1 ? b & 1 : 0], valid, v0, v1);
+                            round_f32_block(vf[kDq == 1 ? b & 1 : 0], ok, v0, v1);
                             vt_write(vt, b - vb0, q, prow, v0, v1);
                         } else {
                             vt_write(vt, b - vb0, q, prow, a0, a1);
@@ -1089,6 +1102,8 @@ __global__ __launch_bounds__(256) void decode_f32_kernel(const DecodeArgs A) {
             });
             __syncthreads();   // V^T tile complete
             pv_tile(vt, pf, j, q, S);
+            ok0 = next0;
+            ok1 = next1;
         }
         emit_partial(A, (long long)blockIdx.x * A.s_max + slot_s, wave, j, q, head, p, 64 * vb0, S);
         ++slot_s;
@@ -2828,7 +2843,7 @@ int launch(DecodeArgs &A, const Plan &pl, hipStream_t st, int phases = 3,
         else if (pl.n_wg * 4 <= num_cus()) {
             // few chunks: four workgroups each, as long as every one has a CU of its
             // own (its registers fill one). On both sides of the line, one against
-            // four: 4096 rows 40.4 -> 36.1 us, 4224 rows 40.5 -> 58.
+            // four: 4096 rows 38.2 -> 35.1 us, 4224 rows 38.4 -> 56.8.
             if (A.f32_v_raw)
                 hipLaunchKernelGGL((decode_f32_kernel<true, 4>), dim3(pl.n_wg, 4), dim3(256), 0, st, A);
             else

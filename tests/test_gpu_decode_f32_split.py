@@ -121,3 +121,20 @@ def test_rounding_of_two_tile_chunks(gpu, n):
     got = out.cpu().numpy()
     assert np.median(rel(one, two)) > 2e-5
     assert np.percentile(rel(got, two), 40) <= 3e-6
+
+
+# 4096 rows: the last count whose chunks are shared; tiles without an allowed row
+@pytest.mark.parametrize("n_raw,n_comp", [(128, 1025), (128, 3968), (128, 3969), (0, 9000)])
+def test_sparse_mask(gpu, n_raw, n_comp):
+    q, k, _, sinks = inputs(n_raw + n_comp, 70 + n_comp)
+    allowed = (synth.uniform(71, n_comp, n_comp) < 0.01).astype(np.int32)
+    allowed[-1] = 1
+    dev = k.copy()
+    dev[n_raw:][allowed == 0] = np.inf
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)
+    out = torch.full((64, 512), float("nan"), device=gpu)
+    ops.launch_flash_attn_decode_mixed_f32(t(q), t(dev[:n_raw]) if n_raw else t(dev[:1]), t(dev[n_raw:]), t(allowed),
+                                           t(sinks), out, 64, n_raw, n_comp, 512)
+    torch.cuda.synchronize()
+    keep = np.concatenate([np.ones(n_raw, bool), allowed.astype(bool)])
+    check(out.cpu().numpy(), reference(q, k[keep], k[keep], sinks.astype(np.float64)))
