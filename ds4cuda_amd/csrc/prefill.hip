@@ -291,10 +291,11 @@ __device__ inline void qk_tile(const uint8_t *st, const uint32_t *ka, const half
 
 // Softmax of one tile with the reference fixed (kFirst: set here, from this
 // tile): writes P hi/lo for the wave's two row tiles and accumulates l and the
-// largest growth over the reference.
+// lane's largest score. (The maximum itself, not its growth over the reference:
+// a row whose first tile is all -inf has no growth to add back.)
 template <bool kFirst, bool kPLo>
 __device__ inline void softmax_fixed(const float4_t (*acc)[2], float kq_log2, int key0, int qpos,
-                                     int g, float *m_use, float *l_part, float *grow,
+                                     int g, float *m_use, float *l_part, float *top,
                                      half8_t *hi_out, half8_t *lo_out) {
     const bool edge = key0 + kTile - 1 > qpos;
 #pragma unroll
@@ -314,29 +315,27 @@ __device__ inline void softmax_fixed(const float4_t (*acc)[2], float kq_log2, in
         }
         const float m = m_use[rt];
         half8_t hi, lo;
-        float lsum = 0.0f, gr = grow[rt];
+        float lsum = 0.0f, mx = top[rt];
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float x = s2[kt][r] - m;   // NaN only where both are -inf (nothing visible yet)
-                gr = fmaxf(gr, x);
-                const float p = s2[kt][r] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(x);
+                mx = fmaxf(mx, s2[kt][r]);
+                const float p = s2[kt][r] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(s2[kt][r] - m);
                 const half_t h = (half_t)p;
                 lsum += kPLo ? p : (float)h;
                 hi[4 * kt + r] = h;
                 if (kPLo) lo[4 * kt + r] = (half_t)(p - (float)h);
             }
-        grow[rt] = gr;
+        top[rt] = mx;
         l_part[rt] += lsum;
         hi_out[rt] = hi;
         lo_out[rt] = lo;
     }
 }
 
-// The growth alone, of a pass whose P is not needed any more.
-__device__ inline void grow_only(const float4_t (*acc)[2], float kq_log2, int key0, int qpos, int g,
-                                 const float *m_use, float *grow) {
+// The largest score alone, of a pass whose P is not needed any more.
+__device__ inline void top_only(const float4_t (*acc)[2], float kq_log2, int key0, int qpos, int g, float *top) {
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
@@ -344,7 +343,7 @@ __device__ inline void grow_only(const float4_t (*acc)[2], float kq_log2, int ke
 #pragma unroll
             for (int r = 0; r < 4; ++r)
                 if (key0 + pi_key(16 * kt + 4 * g + r) <= qpos)
-                    grow[rt] = fmaxf(grow[rt], acc[kt][rt][r] * kq_log2 - m_use[rt]);
+                    top[rt] = fmaxf(top[rt], acc[kt][rt][r] * kq_log2);
 }
 
 // One pass over a pair's tiles (or a part of them), software-pipelined with one
@@ -378,11 +377,7 @@ __global__ __launch_bounds__(256) void prefill_kernel(const PrefillArgs A) {
     // this part's tiles [t0, t1)
     const int all_tiles = (n_all + kTile - 1) / kTile, per = (all_tiles + A.parts - 1) / A.parts;
     const int t0 = (slot % A.parts) * per, t1 = min(t0 + per, all_tiles);
-    if (t0 >= t1) {   // a short pair has fewer parts: an empty partial
-        if (tid < kRows) {
-            A.part_ml[(size_t)slot * 2 * kRows + tid] = -INFINITY;
-            A.part_ml[(size_t)slot * 2 * kRows + kRows + tid] = 0.0f;
-        }
+    if (t0 >= t1) {   // a short pair has fewer parts: the merge leaves this one out
         if (tid == 0) A.fail[slot] = 0;
         return;
     }
@@ -394,10 +389,11 @@ __global__ __launch_bounds__(256) void prefill_kernel(const PrefillArgs A) {
     for (int a = 0; a < 8; ++a)
 #pragma unroll
         for (int b = 0; b < 8; ++b) o[a][b] = float4_t{0, 0, 0, 0};
-    float m_use[2], l_part[2] = {0.f, 0.f}, grow[2] = {0.f, 0.f};
+    float m_use[2], l_part[2] = {0.f, 0.f}, top[2] = {-INFINITY, -INFINITY};
     if (kSecond)
 #pragma unroll
-        for (int rt = 0; rt < 2; ++rt) m_use[rt] = A.row_max[(size_t)slot * kRows + 32 * w + 16 * rt + n16];
+        for (int rt = 0; rt < 2; ++rt)
+            m_use[rt] = A.row_max[(size_t)slot * kRows + 32 * w + 16 * rt + n16];
 
     uint32_t ka[2];
 #pragma unroll
@@ -423,7 +419,7 @@ __global__ __launch_bounds__(256) void prefill_kernel(const PrefillArgs A) {
         store_tile(stages[1], tid, R);
         load_raw(A, t0 + 2, n_all, tid, R);
         half8_t hi[2], lo[2];
-        softmax_fixed<!kSecond, kPLo>(acc, A.kq_log2, t0 * kTile, qpos, g, m_use, l_part, grow, hi, lo);
+        softmax_fixed<!kSecond, kPLo>(acc, A.kq_log2, t0 * kTile, qpos, g, m_use, l_part, top, hi, lo);
 #pragma unroll
         for (int rt = 0; rt < 2; ++rt) {
             pb[0][0][2 * w + rt][lane] = hi[rt];
@@ -447,7 +443,7 @@ __global__ __launch_bounds__(256) void prefill_kernel(const PrefillArgs A) {
             store_tile(stages[sn], tid, R);
             load_raw(A, t + 2, n_all, tid, R);
             half8_t hi[2], lo[2];
-            softmax_fixed<false, kPLo>(acc, A.kq_log2, t * kTile, qpos, g, m_use, l_part, grow, hi, lo);
+            softmax_fixed<false, kPLo>(acc, A.kq_log2, t * kTile, qpos, g, m_use, l_part, top, hi, lo);
 #pragma unroll
             for (int rt = 0; rt < 2; ++rt) {
                 pb[pbuf ^ 1][0][2 * w + rt][lane] = hi[rt];
@@ -462,7 +458,7 @@ __global__ __launch_bounds__(256) void prefill_kernel(const PrefillArgs A) {
         }
         if (!kSecond) {
             volatile int *mark = &flag_s[0];
-            if (__any(fmaxf(grow[0], grow[1]) > kLazy) && lane == 0) *mark = 1;
+            if (__any(fmaxf(top[0] - m_use[0], top[1] - m_use[1]) > kLazy) && lane == 0) *mark = 1;
             stop = __builtin_amdgcn_readfirstlane(*mark) != 0;
         }
     }
@@ -475,7 +471,7 @@ __global__ __launch_bounds__(256) void prefill_kernel(const PrefillArgs A) {
             qk_tile(stages[sc], ka, qf, acc);
             store_tile(stages[sn], tid, R);
             load_raw(A, t + 2, n_all, tid, R);
-            grow_only(acc, A.kq_log2, t * kTile, qpos, g, m_use, grow);
+            top_only(acc, A.kq_log2, t * kTile, qpos, g, top);
             const int tmp = sp;
             sp = sc;
             sc = sn;
@@ -491,13 +487,12 @@ __global__ __launch_bounds__(256) void prefill_kernel(const PrefillArgs A) {
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt) {
         const float l = xsum_16_32(l_part[rt]);
-        const float gr = xmax_16_32(grow[rt]);
-        failed |= gr > kLazy;
+        top[rt] = xmax_16_32(top[rt]);
+        failed |= top[rt] - m_use[rt] > kLazy;   // (NaN where both are -inf: no key seen)
         if (g == 0) {
             const int row = 32 * w + 16 * rt + n16;
             fin_s[0][row] = m_use[rt];
             fin_s[1][row] = l;
-            if (!kSecond) A.row_max[(size_t)slot * kRows + row] = m_use[rt] + gr;
         }
     }
     if (!kSecond) {
@@ -509,7 +504,12 @@ __global__ __launch_bounds__(256) void prefill_kernel(const PrefillArgs A) {
         const int4 fl = *reinterpret_cast<const int4 *>(flag_s);
         const bool fail = (fl.x | fl.y | fl.z | fl.w) != 0;
         if (tid == 0) A.fail[slot] = fail ? 1 : 0;
-        if (fail) return;
+        if (fail) {
+            if (g == 0)
+#pragma unroll
+                for (int rt = 0; rt < 2; ++rt) A.row_max[(size_t)slot * kRows + 32 * w + 16 * rt + n16] = top[rt];
+            return;
+        }
     }
     if (A.parts > 1) {
         if (tid < kRows) {
@@ -548,34 +548,33 @@ __global__ __launch_bounds__(256) void prefill_kernel(const PrefillArgs A) {
 
 // The parts of a pair's keys and the sink, per row (query, head): one wave per
 // row half, a lane's four dims over the parts in order. Bound by the partials'
-// reads (2 KB a row and part).
+// reads (2 KB a row and part). A part whose scores are all -inf counts with
+// weight 0 (not left out: an infinite row makes the same dims NaN as unsplit).
 __global__ __launch_bounds__(256) void prefill_merge_kernel(const PrefillArgs A) {
     const int lane = threadIdx.x & 63, unit = blockIdx.x * 4 + (threadIdx.x >> 6);   // row half
     const int row = unit >> 1, qq = row / kH, head = row % kH;
     if (qq >= A.n_q) return;
     const int slot0 = (qq >> 1) * A.parts, r128 = (qq & 1) * kH + head;
     const float *ml = A.part_ml + (size_t)slot0 * 2 * kRows + r128;
-    const float sink = A.sinks[head] * kLog2e;
-    float m = lane < A.parts ? ml[(size_t)lane * 2 * kRows] : -INFINITY;   // parts <= 64: one per lane
-    const float l = lane < A.parts ? ml[(size_t)lane * 2 * kRows + kRows] : 0.0f;
-    float mx = fmaxf(m, sink);
+    // the pair's parts, as the kernel cut them
+    const int n_all = A.n_cached + min((qq | 1) + 1, A.n_q), all_tiles = (n_all + kTile - 1) / kTile;
+    const int per = (all_tiles + A.parts - 1) / A.parts, parts = (all_tiles + per - 1) / per;
+    float m = lane < parts ? ml[(size_t)lane * 2 * kRows] : -INFINITY;   // parts <= 64: one per lane
+    const float l = lane < parts ? ml[(size_t)lane * 2 * kRows + kRows] : 0.0f;
+    float mx = m;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
     const float sc = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mx);
     float den = l * sc;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) den += __shfl_xor(den, off);
-    den += __builtin_amdgcn_exp2f(sink - mx);
+    const float inv = mx == -INFINITY ? 0.0f : 1.0f / (den + __builtin_amdgcn_exp2f(A.sinks[head] * kLog2e - mx));
     const int d = (unit & 1) * (kD / 2) + 4 * lane;
     const float *po = A.part_o + ((size_t)slot0 * kRows + r128) * kD + d;
     float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 8
-    for (int i = 0; i < A.parts; ++i) {
-        const float c = __shfl(sc, i);
-        const float4_t o = *reinterpret_cast<const float4_t *>(po + (size_t)i * kRows * kD);
-        acc = c != 0.0f ? acc + o * c : acc;   // a select: an empty part's partial was never written
-    }
-    *reinterpret_cast<float4_t *>(A.out + ((size_t)qq * kH + head) * kD + d) = acc * (1.0f / den);
+    for (int i = 0; i < parts; ++i) acc += *reinterpret_cast<const float4_t *>(po + (size_t)i * kRows * kD) * __shfl(sc, i);
+    *reinterpret_cast<float4_t *>(A.out + ((size_t)qq * kH + head) * kD + d) = acc * inv;
 }
 
 // Parts of every pair's keys: as many as fill kSplitWgs workgroups, of at

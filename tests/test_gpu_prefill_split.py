@@ -72,3 +72,23 @@ def test_prefill_workspace_of_another_size(gpu):
         if rc == 0:
             for t in range(n_q):
                 check(out[t].cpu().numpy(), ref[t])
+
+
+# one part and several; the infinite rows: the first tile, and more than a part
+@pytest.mark.parametrize("exact_p", [False, True])
+@pytest.mark.parametrize("n_cached,n_q,n_inf", [(400, 260, 32), (1000, 2, 32), (1000, 5, 300), (1000, 2, 33)])
+def test_prefill_infinite_rows(gpu, n_cached, n_q, n_inf, exact_p):
+    """Rows that are +inf in one dim score -inf for the heads whose query is
+    negative there: they take no weight, and only that dim of the output, where
+    0 * inf is NaN, shows them."""
+    cache, (codes, sexp, tail) = make_cache(n_cached + n_q, 51, gpu)
+    cache.tail[:n_inf, 7] = 0x7C00
+    bits, qf = q_bf16(52, n_q)
+    sinks = sinks_for(53, 1)[0]
+    got = run(gpu, cache, bits, sinks, n_q, n_cached, exact_p=exact_p)
+    ref = oracle_prefill(qf, codes[n_inf:], sexp[n_inf:], tail[n_inf:], n_cached - n_inf, sinks)
+    rest = np.arange(512) != 448 + 7
+    for t in range(n_q):
+        neg = qf[t, :, 448 + 7] < 0
+        assert np.isnan(got[t][neg][:, 448 + 7]).all()
+        check(got[t][neg][:, rest], ref[t][neg][:, rest])
