@@ -34,6 +34,7 @@ SIGNATURES: dict[str, list] = {
         _vp, _i, _ll, _vp, _ll, _vp, _ll, _vp, _vp, _vp, _vp, _i, _vp, _ll, _vp, _ll, _vp, _i,
         _i, _i, _i, _i, _ll, _vp, _vp, _sz, _i, _vp],
     "ds4hip_flash_attn_prefill_fp8_workspace_size": [_i],
+    "ds4hip_flash_attn_prefill_fp8_workspace_for": [_i, _i],
     "ds4hip_flash_attn_prefill_fp8": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, _sz, _i,
                                       _vp],
     "ds4hip_tail_rope_yarn_f32": [_vp, _vp, _i, _i, _i, _i, _i, _vp],
@@ -112,6 +113,7 @@ SIGNATURES: dict[str, list] = {
 # entry points that return a value rather than a status
 RESTYPES = {"ds4hip_indexer_select_scratch_bytes": C.c_size_t,
             "ds4hip_flash_attn_prefill_fp8_workspace_size": C.c_size_t,
+            "ds4hip_flash_attn_prefill_fp8_workspace_for": C.c_size_t,
             "ds4hip_session_state_arena_bytes": C.c_size_t,
             "ds4hip_session_chunk_step_workspace_bytes": C.c_size_t,
             "ds4hip_mul_mm_workspace_bytes": C.c_size_t,

@@ -76,7 +76,6 @@ struct PrefillArgs {
     const int8_t *sexp;
     const uint16_t *tail;
     int *fail;           // [pairs x parts] slots the first pass could not finish
-    float *row_max;      // [pairs x parts][128] their rows' maxima
     float *part_o;       // [pairs x parts][128][512] unnormalized partials (parts > 1)
     float *part_ml;      // [pairs x parts][2][128] their references and sums
     int parts;
@@ -84,6 +83,13 @@ struct PrefillArgs {
     int n_cached;
     float kq_log2;
 };
+
+// Where the first pass leaves a row's maximum for the second: in the slot's own
+// results, which a slot that could not be finished has not written.
+__device__ inline float *row_max_at(const PrefillArgs &A, int slot, int q0, int row) {
+    return A.parts > 1 ? A.part_ml + (size_t)slot * 2 * kRows + row
+                       : A.out + ((long long)(q0 + (row >> 6)) * kH + (row & 63)) * kD;
+}
 
 // Tile-local key of S^T row / P column `idx` (0..31).
 __device__ inline int pi_key(int idx) {
@@ -393,7 +399,7 @@ __global__ __launch_bounds__(256) void prefill_kernel(const PrefillArgs A) {
     if (kSecond)
 #pragma unroll
         for (int rt = 0; rt < 2; ++rt)
-            m_use[rt] = A.row_max[(size_t)slot * kRows + 32 * w + 16 * rt + n16];
+            m_use[rt] = q_ok ? *row_max_at(A, slot, q0, 32 * w + 16 * rt + n16) : -INFINITY;
 
     uint32_t ka[2];
 #pragma unroll
@@ -505,9 +511,9 @@ __global__ __launch_bounds__(256) void prefill_kernel(const PrefillArgs A) {
         const bool fail = (fl.x | fl.y | fl.z | fl.w) != 0;
         if (tid == 0) A.fail[slot] = fail ? 1 : 0;
         if (fail) {
-            if (g == 0)
+            if (g == 0 && q_ok)
 #pragma unroll
-                for (int rt = 0; rt < 2; ++rt) A.row_max[(size_t)slot * kRows + 32 * w + 16 * rt + n16] = top[rt];
+                for (int rt = 0; rt < 2; ++rt) *row_max_at(A, slot, q0, 32 * w + 16 * rt + n16) = top[rt];
             return;
         }
     }
@@ -586,11 +592,10 @@ int prefill_parts(int n_pairs, long long n_rows) {
 }
 
 size_t up256(size_t b) { return (b + 255) & ~(size_t)255; }
-// fail flags and row maxima per slot, and with a split its partials
+// a flag per slot, and with a split its partials
 size_t prefill_ws_bytes(size_t slots, bool split) {
-    size_t b = up256(slots * sizeof(int)) + up256(slots * kRows * sizeof(float));
-    if (split) b += up256(slots * 2 * kRows * sizeof(float)) + slots * kRows * kD * sizeof(float);
-    return b;
+    if (!split) return slots * sizeof(int);
+    return up256(slots * sizeof(int)) + up256(slots * 2 * kRows * sizeof(float)) + slots * kRows * kD * sizeof(float);
 }
 
 }  // namespace
@@ -598,6 +603,12 @@ size_t prefill_ws_bytes(size_t slots, bool split) {
 extern "C" size_t ds4hip_flash_attn_prefill_fp8_workspace_size(int n_q) {
     // a split has at most kSplitWgs slots: enough for it and for one part a pair
     return n_q > 0 ? std::max(prefill_ws_bytes(((size_t)n_q + 1) / 2, false), prefill_ws_bytes(kSplitWgs, true)) : 0;
+}
+
+extern "C" size_t ds4hip_flash_attn_prefill_fp8_workspace_for(int n_q, int n_cached) {
+    if (n_q <= 0 || n_cached < 0) return 0;
+    const int n_pairs = n_q / 2 + (n_q & 1), parts = prefill_parts(n_pairs, (long long)n_cached + n_q);
+    return prefill_ws_bytes((size_t)n_pairs * parts, parts > 1);
 }
 
 extern "C" int ds4hip_flash_attn_prefill_fp8(const void *q, const float *sinks, float *out,
@@ -621,13 +632,13 @@ extern "C" int ds4hip_flash_attn_prefill_fp8(const void *q, const float *sinks, 
     A.sexp = sexp;
     A.tail = tail;
     A.parts = prefill_parts(n_pairs, (long long)n_cached + n_q);
-    if (workspace_bytes < prefill_ws_bytes((size_t)n_pairs * A.parts, A.parts > 1)) A.parts = 1;
+    if (workspace_bytes < prefill_ws_bytes((size_t)n_pairs * A.parts, A.parts > 1) ||
+        (reinterpret_cast<uintptr_t>(workspace) & 15))   // the partials are read 16 bytes at a time
+        A.parts = 1;
     const size_t slots = (size_t)n_pairs * A.parts;
     char *c = static_cast<char *>(workspace);
     A.fail = reinterpret_cast<int *>(c);
     c += up256(slots * sizeof(int));
-    A.row_max = reinterpret_cast<float *>(c);
-    c += up256(slots * kRows * sizeof(float));
     A.part_ml = reinterpret_cast<float *>(c);
     c += up256(slots * 2 * kRows * sizeof(float));
     A.part_o = reinterpret_cast<float *>(c);

@@ -277,7 +277,7 @@ def flash_attn_prefill_fp8(q, sinks, out, cache: Fp8KVCache, n_q, n_cached, row0
     s = cache.sexp[row0:]
     t = cache.tail[row0:]
     from ._lib import lib
-    need = lib().ds4hip_flash_attn_prefill_fp8_workspace_size(n_q)
+    need = lib().ds4hip_flash_attn_prefill_fp8_workspace_for(n_q, n_cached)
     if workspace is None or workspace.numel() < need:
         workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=q.device)
     call("ds4hip_flash_attn_prefill_fp8", _ptr(q), _ptr(sinks), _ptr(out), _ptr(c), _ptr(s),

@@ -235,15 +235,19 @@ long long ds4hip_flash_attn_q_prep_words(void);
  * q [n_q][64][512] bf16 bits, sinks [64] fp32, out [n_q][64][512] fp32;
  * codes/sexp/tail point at the sequence's row 0. workspace holds
  * ds4hip_flash_attn_prefill_fp8_workspace_size(n_q) bytes, a size that also
- * serves every smaller n_q (the partials of a small chunk, whose keys are split
- * over workgroups; flags and row maxima of the query pairs whose softmax range
- * outgrows the first pass, which a second one in the same call redoes). With
- * less, down to 516 bytes per query pair and 512 more, the keys are not split.
+ * serves every smaller n_q: the partials of a small chunk, whose keys are split
+ * over workgroups, and a flag per query pair (two queries, the last one may be
+ * alone) whose softmax range outgrows the first pass, which a second one in the
+ * same call redoes. With less, down to 4 bytes per pair, or at an address that
+ * is not 16-byte aligned, the keys are not split.
+ * ds4hip_flash_attn_prefill_fp8_workspace_for gives what one call can use: 4
+ * bytes per pair where it would not split them (always above 256 queries).
  * exact_p: 0 passes P to the P . V
  * MFMAs as one f16 (l sums the rounded values, so each output stays an exactly
  * normalized average), 1 as f16 hi + lo halves (~22 bits, twice the P . V
  * MFMAs). Per call; nothing is process-wide. */
 size_t ds4hip_flash_attn_prefill_fp8_workspace_size(int n_q);
+size_t ds4hip_flash_attn_prefill_fp8_workspace_for(int n_q, int n_cached);
 int ds4hip_flash_attn_prefill_fp8(const void *q, const float *sinks, float *out,
                                   const uint8_t *codes, const int8_t *sexp, const uint16_t *tail,
                                   int n_q, int n_cached, int n_head, int head_dim, int n_rot,

@@ -119,3 +119,18 @@ def test_bench_and_entry_points_compile():
     import py_compile
     for f in ("bench.py", "__graft_entry__.py"):
         py_compile.compile(str(ROOT / f), doraise=True)
+
+
+def test_prefill_workspace_for_a_call():
+    """What one call can use: a flag per query pair where its keys are not
+    split, never more than the size that serves every smaller chunk."""
+    from ds4cuda_amd import lib
+    l = lib()
+    assert [l.ds4hip_flash_attn_prefill_fp8_workspace_for(n, 100000) for n in (257, 258, 2047, 2048)] == \
+        [4 * 129, 4 * 129, 4 * 1024, 4 * 1024]
+    assert l.ds4hip_flash_attn_prefill_fp8_workspace_for(0, 10) == 0
+    for n_q in (1, 2, 3, 64, 255, 256, 300):
+        size = l.ds4hip_flash_attn_prefill_fp8_workspace_size(n_q)
+        for n_cached in (0, 100, 300, 1000, 8192, 131072):
+            need = l.ds4hip_flash_attn_prefill_fp8_workspace_for(n_q, n_cached)
+            assert 4 * ((n_q + 1) // 2) <= need <= size

@@ -48,7 +48,7 @@ def test_prefill_late_maximum(gpu, n_cached, n_q):
 
 def test_prefill_workspace_of_another_size(gpu):
     """A workspace sized for a large chunk serves a small one (split), and one
-    with room for the flags alone runs it unsplit: the same outputs."""
+    with room for the flags alone (four bytes a pair) runs it unsplit: the same outputs."""
     import ctypes as C
 
     from ds4cuda_amd._lib import lib
@@ -62,7 +62,7 @@ def test_prefill_workspace_of_another_size(gpu):
     ref = oracle_prefill(qf, codes, sexp, tail, n_cached, sinks)
     q = torch.from_numpy(bits.view(np.int16)).to(gpu).view(torch.bfloat16)
     s = torch.from_numpy(np.ascontiguousarray(sinks, np.float32)).to(gpu)
-    for nb, rc in ((size(4096), 0), (3 * 516 + 512, 0), (256, -22)):
+    for nb, rc in ((size(4096), 0), (3 * 516 + 512, 0), (12, 0), (11, -22)):
         out = torch.full((n_q, 64, 512), float("nan"), device=gpu)
         ws = torch.empty(nb, dtype=torch.uint8, device=gpu)
         assert lib().ds4hip_flash_attn_prefill_fp8(
@@ -72,6 +72,36 @@ def test_prefill_workspace_of_another_size(gpu):
         if rc == 0:
             for t in range(n_q):
                 check(out[t].cpu().numpy(), ref[t])
+
+
+@pytest.mark.parametrize("n_cached,n_q", [(1000, 3), (400, 259)])
+def test_prefill_late_maximum_with_flags_only(gpu, n_cached, n_q):
+    """The smallest workspace holds no row maxima: a pair that the first pass
+    gives up is redone all the same, here the first and (odd) last ones."""
+    import ctypes as C
+
+    from ds4cuda_amd import ops
+    from ds4cuda_amd._lib import lib
+    from ds4cuda_amd.ops import _ptr, _stream
+    bits, qf = q_bf16(45, n_q)
+    x = synth.kv_rows(44, 0, n_cached + n_q)
+    x[n_cached - 1] = 6.0 * qf[0, 5]
+    x[n_cached - 2] = 6.0 * qf[n_q - 1, 60]
+    cache = ops.Fp8KVCache.empty(n_cached + n_q, device=gpu)
+    cache.append(torch.from_numpy(x).to(gpu))
+    sinks = sinks_for(46, 1)[0]
+    q = torch.from_numpy(bits.view(np.int16)).to(gpu).view(torch.bfloat16)
+    s = torch.from_numpy(np.ascontiguousarray(sinks, np.float32)).to(gpu)
+    out = torch.full((n_q, 64, 512), float("nan"), device=gpu)
+    ws = torch.empty(4 * ((n_q + 1) // 2), dtype=torch.uint8, device=gpu)
+    assert lib().ds4hip_flash_attn_prefill_fp8(
+        _ptr(q), _ptr(s), _ptr(out), _ptr(cache.codes), _ptr(cache.sexp), _ptr(cache.tail), n_q, n_cached, 64, 512, 64,
+        _ptr(ws), C.c_size_t(ws.numel()), 0, _stream(None)) == 0
+    torch.cuda.synchronize()
+    ref = oracle_prefill(qf, cache.codes.cpu().numpy(), cache.sexp.cpu().numpy(),
+                         cache.tail.cpu().numpy().view(np.uint16), n_cached, sinks)
+    for t in range(n_q):
+        check(out[t].cpu().numpy(), ref[t])
 
 
 # one part and several; the infinite rows: the first tile, and more than a part
