@@ -134,3 +134,14 @@ def test_prefill_workspace_for_a_call():
         for n_cached in (0, 100, 300, 1000, 8192, 131072):
             need = l.ds4hip_flash_attn_prefill_fp8_workspace_for(n_q, n_cached)
             assert 4 * ((n_q + 1) // 2) <= need <= size
+
+
+def test_prefill_split_where_it_pays():
+    """Keys are split over workgroups only where the tiles saved outweigh the
+    partials: not for 128 to 255 queries over a few hundred rows."""
+    from ds4cuda_amd import lib
+
+    def split(n_q, n_cached):
+        return lib().ds4hip_flash_attn_prefill_fp8_workspace_for(n_q, n_cached) > 4 * ((n_q + 1) // 2)
+    assert not any(split(n_q, c) for n_q, c in ((255, 0), (255, 128), (200, 128), (128, 128), (96, 32), (1, 32)))
+    assert all(split(n_q, c) for n_q, c in ((255, 250), (255, 400), (200, 400), (128, 250), (64, 400), (2, 400), (1, 8000)))
