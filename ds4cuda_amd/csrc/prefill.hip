@@ -367,7 +367,7 @@ __global__ __launch_bounds__(256) void prefill_kernel(const PrefillArgs A) {
     __shared__ __attribute__((aligned(16))) uint8_t stages[3][kStageB];
     __shared__ __attribute__((aligned(16))) half8_t pb[2][2][8][64];   // [buf][hi,lo][row tile][lane]
     __shared__ __attribute__((aligned(16))) int flag_s[4];
-    __shared__ __attribute__((aligned(16))) float fin_s[2][kRows];
+    __shared__ __attribute__((aligned(16))) float fin_s[3][kRows];
 
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int n16 = lane & 15, g = lane >> 4;
@@ -399,7 +399,8 @@ __global__ __launch_bounds__(256) void prefill_kernel(const PrefillArgs A) {
     if (kSecond)
 #pragma unroll
         for (int rt = 0; rt < 2; ++rt)
-            m_use[rt] = q_ok ? *row_max_at(A, slot, q0, 32 * w + 16 * rt + n16) : -INFINITY;
+            // (the missing second query of a last pair sees no key: any reference does)
+            m_use[rt] = *row_max_at(A, slot, q0, (q_ok ? 32 * w : 32 * (w & 1)) + 16 * rt + n16);
 
     uint32_t ka[2];
 #pragma unroll
@@ -499,6 +500,7 @@ __global__ __launch_bounds__(256) void prefill_kernel(const PrefillArgs A) {
             const int row = 32 * w + 16 * rt + n16;
             fin_s[0][row] = m_use[rt];
             fin_s[1][row] = l;
+            if (!kSecond) fin_s[2][row] = top[rt];
         }
     }
     if (!kSecond) {
@@ -511,9 +513,7 @@ __global__ __launch_bounds__(256) void prefill_kernel(const PrefillArgs A) {
         const bool fail = (fl.x | fl.y | fl.z | fl.w) != 0;
         if (tid == 0) A.fail[slot] = fail ? 1 : 0;
         if (fail) {
-            if (g == 0 && q_ok)
-#pragma unroll
-                for (int rt = 0; rt < 2; ++rt) *row_max_at(A, slot, q0, 32 * w + 16 * rt + n16) = top[rt];
+            if (tid < kRows && q0 + (tid >> 6) < A.n_q) *row_max_at(A, slot, q0, tid) = fin_s[2][tid];
             return;
         }
     }
@@ -588,9 +588,11 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const PrefillArgs A)
 // workgroup saves (1.85 us each) outweigh the partials (2 us, and 0.05 for the
 // 256 KB that a slot writes and the merge reads). Measured over 1 to 255
 // queries x 0 to 8000 rows, unsplit and split: 128 queries over 128 rows
-// 35.4 / 35.6 us (not split), over 250 42.6 / 39.1; 255 over 0 36.8 / 42.9 and
-// over 128 44.7 / 48.9 (not split), over 250, on the line, 51.9 / 52.9, over 400
-// 60.7 / 58.0.
+// 33.7 / 34.5 us (not split), over 250 40.9 / 38.5; 255 over 0 34.8 / 42.4 and
+// over 128 42.2 / 48.3 (not split), over 400 58.4 / 57.4. The line is drawn at
+// 255 over 250 (16 tiles, 49.5 / 52.4), which still splits: P, one f16 relative
+// to its part's first maximum, errs less in a shorter part (2.1e-3 of the
+// output's RMS at most unsplit there).
 int prefill_parts(int n_pairs, long long n_rows) {
     const long long tiles = (n_rows + kTile - 1) / kTile;
     const long long parts = std::min<long long>({kSplitWgs / n_pairs, tiles / kMinPartTiles, kMaxParts});
