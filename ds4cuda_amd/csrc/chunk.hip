@@ -367,11 +367,12 @@ ChunkWs chunk_ws(void *base, int n, int ratio, int cap_keys) {
         W.iscore = take((size_t)n * 2 * kIdxDim);
         W.q_idx = take((size_t)n * kIdxHeads * kIdxDim);
         W.w_idx = take((size_t)n * kIdxHeads);
-        // past the chunk selection's key limit the tokens select one by one
-        const bool together = cap_keys <= ds4hip_indexer_chunk_max_keys();
-        W.score_stride = (cap_keys + 63) & ~63;
-        W.scores = take((size_t)(together ? n : 1) * W.score_stride);
-        if (!together) W.select = reinterpret_cast<uint8_t *>(take(ds4hip_indexer_select_scratch_bytes(cap_keys) / 4 + 1));
+        // tokens past the chunk selection's key limit select one by one, with
+        // the same scratch (in stream order) for their scores
+        W.score_stride = (std::min(cap_keys, ds4hip_indexer_chunk_max_keys()) + 63) & ~63;
+        W.scores = take(std::max((size_t)n * W.score_stride, (size_t)cap_keys));
+        if (cap_keys > ds4hip_indexer_chunk_max_keys())
+            W.select = reinterpret_cast<uint8_t *>(take(ds4hip_indexer_select_scratch_bytes(cap_keys) / 4 + 1));
     }
     W.bytes = off;
     return W;
@@ -461,22 +462,23 @@ int chunk_step(ds4hip_session_state *s, int il, int p0, int n, const float *attn
                                             L->row_base + L->n_comp, nullptr, st)))
         return rc;
     const int n_idx0 = L->n_index_comp;
+    auto keys_of = [&](int t) { return n_idx0 + (p0 + t + 1) / ratio - p0 / ratio; };
     for (int t = 0; t < n; ++t) {
-        const int e = (p0 + t + 1) / ratio - p0 / ratio;
-        n_comp_tok[t] = n_sel_tok[t] = L->n_comp + e;
-        if (idx && n_idx0 + e > w->top_k) n_sel_tok[t] = w->top_k;
+        n_comp_tok[t] = n_sel_tok[t] = L->n_comp + (p0 + t + 1) / ratio - p0 / ratio;
+        if (idx && keys_of(t) > w->top_k) n_sel_tok[t] = w->top_k;
     }
-    if (select && !W.select) {
-        rc = ds4hip_indexer_chunk_topk(W.q_idx, W.w_idx, L->index_comp_kv, n, p0, ratio, n_idx0, kIdxHeads, w->top_k,
-                                       W.scores, W.score_stride, sel, st);
-    } else if (select) {
-        for (int t = 0; t < n && !rc; ++t) {
-            const int keys = n_idx0 + (p0 + t + 1) / ratio - p0 / ratio;
-            if (keys > w->top_k)
+    if (select) {
+        // the keys a token sees, not those the session could hold, decide its form
+        int together = 0;
+        while (together < n && keys_of(together) <= ds4hip_indexer_chunk_max_keys()) ++together;
+        if (together)
+            rc = ds4hip_indexer_chunk_topk(W.q_idx, W.w_idx, L->index_comp_kv, together, p0, ratio, n_idx0, kIdxHeads,
+                                           w->top_k, W.scores, W.score_stride, sel, st);
+        for (int t = together; t < n && !rc; ++t)
+            if (keys_of(t) > w->top_k)
                 rc = ds4hip_indexer_topk_positions(W.q_idx + (size_t)t * kIdxHeads * kIdxDim, W.w_idx + (size_t)t * kIdxHeads,
-                                                   L->index_comp_kv, 0, keys, kIdxHeads, kIdxDim, w->top_k, 0, W.scores,
-                                                   W.select, nullptr, sel + (size_t)t * w->top_k, st);
-        }
+                                                   L->index_comp_kv, 0, keys_of(t), kIdxHeads, kIdxDim, w->top_k, 0,
+                                                   W.scores, W.select, nullptr, sel + (size_t)t * w->top_k, st);
     }
     if (rc) return rc;
     L->n_comp += n_emit;
