@@ -60,12 +60,10 @@ __device__ inline float key_elem(const void *keys, size_t i) {
 }
 
 // The reference's head sum (see the top of the file), fed one leaf at a time
-// in leaf order: leaf t of warp t >> kLevels. A leaf is one head's product
-// (kLevels = 5) or the sum of a group of four heads h, h + 16, h + 8, h + 24
-// (kLevels = 3, the butterfly's first two levels already added). An odd leaf
-// index closes a pair with the level below, like a binary counter's carry.
-template <int kLevels>
+// in leaf order: leaf t, one head's product, of warp t / 32. An odd leaf index
+// closes a pair with the level below, like a binary counter's carry.
 struct HeadTree {
+    static constexpr int kLevels = 5;
     float l[kLevels];
     float w0 = 0.0f, w1 = 0.0f;
     // branch-free (t is uniform, but branches here cost the caller's
@@ -171,7 +169,7 @@ struct ScoreSeq {
 // Scores keys [c0, end) of one sequence by a workgroup of four waves, 16 a
 // time: wave t takes heads 16 t .. 16 t + 15 (32 registers of query operands
 // and one accumulator), and the products meet in LDS for the tree. Heads past
-// n_head read head 0 and add +0.0f, as the reference's idle threads do.
+// n_head read the last one's query and add +0.0f, as the reference's idle threads do.
 // store(key, score) is called by the lane that finished the key.
 //
 // What bounds it: the fp32 matrix rate, 15 ns per 16 keys x 16 heads x 4 dims
@@ -274,7 +272,7 @@ __device__ inline float score_any(const float *qs, const float *ws, const void *
 #pragma unroll
     for (int d = 0; d < kMaxDim; ++d)
         k[d] = d < head_dim ? key_elem<kKind>(keys, (size_t)c * head_dim + d) : 0.0f;
-    HeadTree<5> tree;
+    HeadTree tree;
     const int n_leaves = (n_head + 31) & ~31;
     for (int t = 0; t < n_leaves; ++t) {
         const int h = head_of_leaf(t);
@@ -626,8 +624,8 @@ int score_select(const float *q, const float *w, const void *keys, int kind, int
     const int recent = n_recent < top_k ? n_recent : top_k;
     const int n_cand = n_comp - recent;
     // Few candidates and positions only (the model's decode: a few thousand
-    // compressed rows): the batched pair with one sequence, four lanes per
-    // key and one workgroup's LDS radix select, two launches instead of six;
+    // compressed rows): the batched pair with one sequence, the scores and
+    // one workgroup's LDS radix select, two launches instead of six;
     // the same scores and the same selection rule.
     if (!mask && head_dim == kMaxDim && n_cand <= kSmallSelect) {
         const long long row0 = 0;
