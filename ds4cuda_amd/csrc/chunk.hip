@@ -50,7 +50,9 @@ constexpr int kIdxHeads = 64, kIdxDim = DS4HIP_INDEXER_HEAD_DIM;
 // 16 (three waves per SIMD, half as much again from L2), 115 us with 16 x 32,
 // 230 us with 32 x 32 (one wave per SIMD); one matvec launch per token and
 // matrix took 21 us a token. Up to 16 tokens take 16 x 16, where twice the
-// workgroups stream the weights.
+// workgroups stream the weights; the line is a token tile's. Whole chunks with
+// 32 and 16 rows: 16 tokens without a selection 68.0 and 66.7 us, with one 90.1
+// and 92.3; 17 tokens 99.2 and 104.1, 64 tokens 141.7 and 149.9.
 
 __device__ inline void lanes_to_steps(uint32_t (&v)[4]) {
     // lane group g holds v[i] of chain g; afterwards v[j] of group g is
@@ -81,32 +83,29 @@ struct ProjArgs {
 };
 
 // A lane's raw pieces of one step of the pipeline: its row's eight f16 weights
-// per row tile and its token's eight inputs per token tile.
-template <int kR, int kT>
+// per row tile and its token's eight inputs.
+template <int kR>
 struct Pieces {
     uint4_t w[kR];
-    float4_t x[kT][2];
-    __device__ inline void load(const uint16_t *const (&wp)[kR], const float *const (&xp)[kT], bool x_wide, int e0) {
+    float4_t x[2];
+    __device__ inline void load(const uint16_t *const (&wp)[kR], const float *xp, bool x_wide, int e0) {
 #pragma unroll
         for (int r = 0; r < kR; ++r) w[r] = *reinterpret_cast<const uint4_t *>(wp[r] + e0);
+        const float *p = xp + e0;
 #pragma unroll
-        for (int t = 0; t < kT; ++t) {
-            const float *p = xp[t] + e0;
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-                x[t][h] = x_wide ? *reinterpret_cast<const float4_t *>(p + 4 * h)
-                                 : float4_t{p[4 * h], p[4 * h + 1], p[4 * h + 2], p[4 * h + 3]};
-        }
+        for (int h = 0; h < 2; ++h)
+            x[h] = x_wide ? *reinterpret_cast<const float4_t *>(p + 4 * h)
+                          : float4_t{p[4 * h], p[4 * h + 1], p[4 * h + 2], p[4 * h + 3]};
     }
 };
 
-// One wave's chains of a (16 kR) x (16 kT) tile: kJ pieces per chain. sum[i]:
+// One wave's chains of a (16 kR) x 16 tile: kJ pieces per chain. sum[i]:
 // chains i of its four groups added (offsets 32, 16). x_wide: x is 16-byte
 // aligned (else four 4-byte loads). The pieces are loaded two steps ahead:
 // with two waves per SIMD nothing else covers the L2 latency.
-template <int kJ, int kR, int kT>
-__device__ inline void chain_tiles(const uint16_t *const (&w)[kR], const float *const (&x)[kT], bool x_wide, int wave,
-                                   float4_t (&sum)[4][kR][kT]) {
+template <int kJ, int kR>
+__device__ inline void chain_tiles(const uint16_t *const (&w)[kR], const float *x, bool x_wide, int wave,
+                                   float4_t (&sum)[4][kR]) {
     static_assert(kJ % 2 == 0, "the two buffers alternate by piece");
     const int g = (threadIdx.x & 63) >> 4;
     // step q = kJ s + j: piece j of group s, groups in the order w, w + 8, w + 4, w + 12
@@ -114,23 +113,21 @@ __device__ inline void chain_tiles(const uint16_t *const (&w)[kR], const float *
         const int sq = (q / kJ) & 3, j = q % kJ;
         return (4 * (wave + ((sq & 1) << 3) + ((sq >> 1) << 2)) + g + 64 * j) * 8;
     };
-    float4_t half[4][kR][kT];
-    Pieces<kR, kT> buf[2];
+    float4_t half[4][kR];
+    Pieces<kR> buf[2];
     buf[0].load(w, x, x_wide, elem(0));
     buf[1].load(w, x, x_wide, elem(1));
 #pragma unroll 1
     for (int s = 0; s < 4; ++s) {
-        float4_t acc[4][kR][kT];
+        float4_t acc[4][kR];
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int r = 0; r < kR; ++r)
-#pragma unroll
-                for (int t = 0; t < kT; ++t) acc[i][r][t] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int r = 0; r < kR; ++r) acc[i][r] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int j = 0; j < kJ; ++j) {
-            Pieces<kR, kT> &cur = buf[j & 1];
-            uint32_t a[kR][2][4], b[kT][2][4];
+            Pieces<kR> &cur = buf[j & 1];
+            uint32_t a[kR][2][4], b[2][4];
 #pragma unroll
             for (int r = 0; r < kR; ++r)
 #pragma unroll
@@ -138,47 +135,40 @@ __device__ inline void chain_tiles(const uint16_t *const (&w)[kR], const float *
                     a[r][e >> 2][e & 3] =
                         __float_as_uint(f16_bits_to_f32((uint16_t)((cur.w[r][e >> 1] >> (16 * (e & 1))) & 0xFFFF)));
 #pragma unroll
-            for (int t = 0; t < kT; ++t)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) b[t][e >> 2][e & 3] = __float_as_uint(cur.x[t][e >> 2][e & 3]);
+            for (int e = 0; e < 8; ++e) b[e >> 2][e & 3] = __float_as_uint(cur.x[e >> 2][e & 3]);
             cur.load(w, x, x_wide, elem(kJ * s + j + 2));   // past the last step: group 0 again, unused
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
 #pragma unroll
                 for (int r = 0; r < kR; ++r) lanes_to_steps(a[r][h]);
-#pragma unroll
-                for (int t = 0; t < kT; ++t) lanes_to_steps(b[t][h]);
+                lanes_to_steps(b[h]);
 #pragma unroll
                 for (int r = 0; r < kR; ++r)
 #pragma unroll
-                    for (int t = 0; t < kT; ++t)
-#pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            acc[i][r][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                                __uint_as_float(a[r][h][i]), __uint_as_float(b[t][h][i]), acc[i][r][t], 0, 0, 0);
+                    for (int i = 0; i < 4; ++i)
+                        acc[i][r] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a[r][h][i]),
+                                                                         __uint_as_float(b[h][i]), acc[i][r], 0, 0, 0);
             }
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int r = 0; r < kR; ++r)
-#pragma unroll
-                for (int t = 0; t < kT; ++t) {
-                    if (s == 0) sum[i][r][t] = acc[i][r][t];
-                    if (s == 1) sum[i][r][t] = sum[i][r][t] + acc[i][r][t];
-                    if (s == 2) half[i][r][t] = acc[i][r][t];
-                    if (s == 3) sum[i][r][t] = sum[i][r][t] + (half[i][r][t] + acc[i][r][t]);
-                }
+            for (int r = 0; r < kR; ++r) {
+                if (s == 0) sum[i][r] = acc[i][r];
+                if (s == 1) sum[i][r] = sum[i][r] + acc[i][r];
+                if (s == 2) half[i][r] = acc[i][r];
+                if (s == 3) sum[i][r] = sum[i][r] + (half[i][r] + acc[i][r]);
+            }
     }
 }
 
-template <int kR, int kT>
+template <int kR>
 __global__ __launch_bounds__(256, 2) void chunk_project_kernel(const ProjArgs A) {
-    __shared__ float red[4][4][kR * kT][4][64];   // [wave][chain][tile][register][lane]
+    __shared__ float red[4][4][kR][4][64];   // [wave][chain][row tile][register][lane]
     // the token tiles of a row tile run on one XCD (workgroups go to the eight
     // in turn), so its L2 reads those weights once: 107 -> 98 us for 128 tokens
-    const int tok_tiles = (A.n + 16 * kT - 1) / (16 * kT);
+    const int tok_tiles = (A.n + 15) / 16;
     const int row_tile = (int)blockIdx.x / (8 * tok_tiles) * 8 + (int)blockIdx.x % 8;
     if (row_tile >= A.blk0[kMaxJobs]) return;
     int jb = 0;
@@ -187,39 +177,35 @@ __global__ __launch_bounds__(256, 2) void chunk_project_kernel(const ProjArgs A)
         if (row_tile >= A.blk0[i]) jb = i;
     const ProjJob J = A.j[jb];
     const int K = J.k_is_lora ? kLora : kEmbd;
-    const int row0 = (row_tile - A.blk0[jb]) * 16 * kR, tok0 = (int)blockIdx.x / 8 % tok_tiles * 16 * kT;
+    const int row0 = (row_tile - A.blk0[jb]) * 16 * kR, tok0 = (int)blockIdx.x / 8 % tok_tiles * 16;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint16_t *w[kR];
-    const float *x[kT];
 #pragma unroll
     for (int r = 0; r < kR; ++r) w[r] = J.w + (size_t)(row0 + 16 * r + (lane & 15)) * K;
-#pragma unroll
-    for (int t = 0; t < kT; ++t) x[t] = J.x + (size_t)min(tok0 + 16 * t + (lane & 15), A.n - 1) * K;
-    float4_t sum[4][kR][kT];
+    const float *x = J.x + (size_t)min(tok0 + (lane & 15), A.n - 1) * K;
+    float4_t sum[4][kR];
     const bool wide = (reinterpret_cast<uintptr_t>(J.x) & 15) == 0;
-    if (J.k_is_lora) chain_tiles<kLora / 512, kR, kT>(w, x, wide, wave, sum);
-    else chain_tiles<kEmbd / 512, kR, kT>(w, x, wide, wave, sum);
+    if (J.k_is_lora) chain_tiles<kLora / 512, kR>(w, x, wide, wave, sum);
+    else chain_tiles<kEmbd / 512, kR>(w, x, wide, wave, sum);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int r = 0; r < kR; ++r)
 #pragma unroll
-            for (int t = 0; t < kT; ++t)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) red[wave][i][r * kT + t][e][lane] = sum[i][r][t][e];
+            for (int e = 0; e < 4; ++e) red[wave][i][r][e][lane] = sum[i][r][e];
     __syncthreads();
-    // wave `wave` finishes register `wave` of every tile: row 4 (lane / 16) +
+    // wave `wave` finishes register `wave` of every row tile: row 4 (lane / 16) +
     // wave, token lane % 16
+    const int tok = tok0 + (lane & 15);
 #pragma unroll
-    for (int tile = 0; tile < kR * kT; ++tile) {
+    for (int r = 0; r < kR; ++r) {
         float c[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            c[i] = (red[0][i][tile][wave][lane] + red[2][i][tile][wave][lane]) +
-                   (red[1][i][tile][wave][lane] + red[3][i][tile][wave][lane]);
+            c[i] = (red[0][i][r][wave][lane] + red[2][i][r][wave][lane]) +
+                   (red[1][i][r][wave][lane] + red[3][i][r][wave][lane]);
         float v = (c[0] + c[2]) + (c[1] + c[3]);
-        const int row = row0 + 16 * (tile / kT) + 4 * (lane >> 4) + wave;
-        const int tok = tok0 + 16 * (tile % kT) + (lane & 15);
+        const int row = row0 + 16 * r + 4 * (lane >> 4) + wave;
         if (tok >= A.n) continue;
         if (J.ape) v = v + f16_bits_to_f32(J.ape[(size_t)((A.p0 + tok) % A.ratio) * J.ld + row]);
         if (J.scale != 1.0f) v = v * J.scale;
@@ -378,10 +364,9 @@ ChunkWs chunk_ws(void *base, int n, int ratio, int cap_keys) {
     return W;
 }
 
-template <int kR, int kT>
+template <int kR>
 void launch_project(const ProjArgs &A, int blocks, hipStream_t st) {
-    hipLaunchKernelGGL((chunk_project_kernel<kR, kT>), dim3((blocks + 7) / 8 * 8 * ((A.n + 16 * kT - 1) / (16 * kT))),
-                       dim3(256), 0, st, A);
+    hipLaunchKernelGGL(chunk_project_kernel<kR>, dim3((blocks + 7) / 8 * 8 * ((A.n + 15) / 16)), dim3(256), 0, st, A);
 }
 
 int chunk_step(ds4hip_session_state *s, int il, int p0, int n, const float *attn_norm, const float *q_lora,
@@ -426,8 +411,8 @@ int chunk_step(ds4hip_session_state *s, int il, int p0, int n, const float *attn
         job(w->idx_q_b, q_lora, W.q_idx, nullptr, 1.0f, kIdxHeads * kIdxDim, 1);
     }
     for (int i = jobs; i <= kMaxJobs; ++i) P.blk0[i] = blk;
-    if (big) launch_project<2, 1>(P, blk, st);
-    else launch_project<1, 1>(P, blk, st);
+    if (big) launch_project<2>(P, blk, st);
+    else launch_project<1>(P, blk, st);
     int rc = hip_status(hipGetLastError());
     if (rc) return rc;
 
