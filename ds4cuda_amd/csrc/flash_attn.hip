@@ -2451,8 +2451,12 @@ __global__ __launch_bounds__(256) void phys_kernel(const DecodeArgs A) {
 //
 // kMany: many workgroups per CU hide each other's loads, so the slots are read
 // one by one without the repeated rows of a short group of eight (43 problems of
-// six chunks 12.0 us, 14.6 in groups); one problem's 64 workgroups are bound by
-// their own chain and code (8.4 us slot by slot, unrolled; 6.9 in groups).
+// 32768 rows, whose partials come from memory, 12.0 us, 14.6 in groups); fewer
+// are bound by their own chain and code. Slot by slot and in groups, 200 rows
+// each: 8 problems 6.3 and 4.7 us, 16 6.3 and 5.5, 24 7.1 and 6.5, 43 alike
+// (7.0). From 32 problems on, a long context's 256 chunks are at most eight per
+// problem, the most this merge takes.
+constexpr int kMergeManyProblems = 32;
 template <bool kMany>
 __global__ __launch_bounds__(128) void decode_merge_kernel(const DecodeArgs A) {
     __shared__ float s_sc[128], s_dl[128];
@@ -2553,11 +2557,12 @@ __global__ __launch_bounds__(128) void decode_merge_kernel(const DecodeArgs A) {
 // slots (slot j to wave j mod 4, in slot order), thread t dims 4t..4t+3 of the
 // half, several slots' 16-byte loads in flight, and the four waves' sums are
 // added in wave order: a fixed order, so the result is deterministic.
-constexpr int kMergeManyProblems = 8;   // 64 merges each: two workgroups per CU
 constexpr int kMergeThreads = 256;
 constexpr long long kMergeWideSlots = 8;   // chunks per problem above which the wide merge runs
-// kMany as above: 16 problems 10.4 us slot by slot, 11.0 in groups; one problem
-// of 20 chunks 8.4 and 7.6.
+// kMany as above. Slot by slot and in groups: one problem of 20 chunks 8.4 and
+// 7.6 us; 4096 rows each, 8 problems 8.4 and 8.2, 12 8.1 and 7.8, 16 8.4 and
+// 9.6, 20 alike (9.9); whole calls 12 problems 28.6 and 28.4, 14 29.1 and 30.2.
+constexpr int kMergeWideManyProblems = 13;
 template <bool kMany>
 __global__ __launch_bounds__(kMergeThreads) void decode_merge_wide_kernel(const DecodeArgs A) {
     __shared__ float s_sc[kMergeThreads];
@@ -2867,7 +2872,7 @@ int launch(DecodeArgs &A, const Plan &pl, hipStream_t st, int phases = 3,
             if (b1 > b0)
                 max_slots = std::max(max_slots, (b1 - 1) / A.chunk - b0 / A.chunk + 1);
         }
-        if (max_slots > kMergeWideSlots && A.n_prob >= kMergeManyProblems)
+        if (max_slots > kMergeWideSlots && A.n_prob >= kMergeWideManyProblems)
             hipLaunchKernelGGL(decode_merge_wide_kernel<true>, dim3(A.n_prob, kH, 2), dim3(kMergeThreads), 0, st, A);
         else if (max_slots > kMergeWideSlots)
             hipLaunchKernelGGL(decode_merge_wide_kernel<false>, dim3(A.n_prob, kH, 2), dim3(kMergeThreads), 0, st, A);

@@ -58,3 +58,19 @@ def test_segments_share_chunks(gpu, counts):
             assert (got[p] == 0).all()
         else:
             check(got[p], O.attn_decode_fp8(qf[p], codes, sexp, tail, base[p] + np.arange(counts[p]), sinks[p]))
+
+
+# more than eight chunks a problem (the wide merge) and fewer, on both sides of
+# the problem counts from which the slots are read one by one
+@pytest.mark.parametrize("n,rows", [(12, 1200), (13, 1200), (31, 300), (32, 300)])
+def test_merge_forms(gpu, n, rows):
+    cache, (codes, sexp, tail) = make_cache(n * rows, 74, gpu)
+    bits, qf = q_bf16(75, n)
+    sinks = sinks_for(76, n)
+    out = torch.full((n, 64, 512), float("nan"), device=gpu)
+    q = torch.from_numpy(bits.view(np.int16)).to(gpu).view(torch.bfloat16)
+    ops.flash_attn_decode_fp8(q, torch.from_numpy(sinks).to(gpu), out, cache, [rows] * n, row_base_stride=rows)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    for p in (0, n // 2, n - 1):
+        check(got[p], O.attn_decode_fp8(qf[p], codes, sexp, tail, p * rows + np.arange(rows), sinks[p]))
