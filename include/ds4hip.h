@@ -396,7 +396,8 @@ int ds4hip_rms_norm_batch_f32(const float *x, const float *w, int weight_dim, fl
 size_t ds4hip_attn_qkv_decode_workspace_bytes(void);
 
 /* The decode Q / KV producer of one layer, Steps 3-10 of
- * cuda/forward_layer.cu:827-913 in one call (six launches, no allocation):
+ * cuda/forward_layer.cu:827-913 in one call (three launches, seven where a weight is not
+ * 16-byte aligned; no allocation):
  *   q_lora      = Q8_0 matvec(w_q_a [1024 x 4096], attn_norm [4096])
  *   q_lora_norm = RMSNorm(q_lora, w_q_a_norm [1024])          -> q_lora_norm
  *   kv_raw      = Q8_0 matvec(w_kv_a [512 x 4096], attn_norm)

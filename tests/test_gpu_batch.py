@@ -140,9 +140,8 @@ def test_compressor_batch_matches_per_sequence(gpu):
 @pytest.mark.parametrize("key_kind", [0, 1, 2])
 def test_indexer_batch_positions(gpu, key_kind, sizes):
     """Batched scorer + selection for fp32 (0), f16 (1) and bf16 (2) keys:
-    scores and positions bit-exact against the oracle per sequence. few: up
-    to 10240 keys scored in all (the lane-per-head scorer); many: more (the
-    four-lane scorer)."""
+    scores and positions bit-exact against the oracle per sequence, for a few
+    thousand keys scored in all (few) and more (many)."""
     n_comp = [100, 512, 513, 2000, 4000, 3] + ([5000, 700] if sizes == "many" else [])
     n_seq, top_k, recent = len(n_comp), 512, 64
     row0 = np.concatenate([[0], np.cumsum(n_comp)[:-1]]) + 10
